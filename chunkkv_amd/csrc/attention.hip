@@ -18,11 +18,10 @@
 // four lane groups. K/V tiles go from global memory straight into double-buffered LDS (no
 // register staging, one barrier per tile), in swizzled rows that make the fragment reads
 // conflict-free; V^T comes out of row-major V through transposing LDS reads. Scores and the output accumulate in
-// fp32; P is rounded to bf16 for the second product (as fused SDPA kernels do). When a launch
-// would have too few workgroups to fill the chip (decode: one query, long cache) the cache range
-// is split over more workgroups (flash-decoding): each writes unnormalised fp32 rows with their
-// running max and sum to a caller-provided workspace, and a small kernel merges the splits. Built with the
-// MFMA VGPR form (no accumulator-register copies around the online-softmax rescale).
+// fp32; P is rounded to bf16 for the second product (as fused SDPA kernels do). Launches with too
+// few 128-query workgroups to fill the chip (decode, short prompts, small blends) run
+// attention_wave.hpp's kernel instead. Built with the MFMA VGPR form (no accumulator-register
+// copies around the online-softmax rescale).
 #include <algorithm>
 
 #include "ckv_common.hpp"
@@ -39,6 +38,7 @@ constexpr int kAttnWaves = 4;
 constexpr int kAttnQG = CKV_ATTN_QG;                // 16-query groups per wavefront
 constexpr int kAttnBM = kAttnWaves * kAttnQG * 16;  // queries per workgroup
 constexpr int kAttnBN = 64;                         // cache rows per tile
+constexpr int kWaveChunk = 32;                      // cache rows per step of attn_wave_kernel's wavefronts
 
 // Combine a lane's value with the lanes 16 and 32 away (the four lane groups of one query), with
 // gfx950's row-swap permutes (VALU, no LDS round trip): each returns the lane's own value and
@@ -79,62 +79,90 @@ __device__ __forceinline__ int kslot_row(int s) {
   return (s & ~31) + 8 * ((k >> 2) & 3) + 4 * (k >> 4) + (k & 3);
 }
 
+// The A operand of O^T = V^T P^T for columns 16 dt .. + 16 of 32 V rows at vb (swizzled, row-major),
+// through transposing 64-bit LDS loads: in each 16-lane group, lane m names row 4 h + m / 4 (of the
+// group's 8 keys 8 g ..) at column 4 (m % 4) of the 16-column tile, and lane 4a + b receives column
+// 4a + b of rows 4h + 0..3. So lane (g, lm) holds V[8 g + 4 h + e][16 dt + lm], e = 0..3: two loads
+// (h = 0, 1) give the eight keys 8 g + e' the B operand (P^T) pairs with that lane. Element
+// 16 dt + 4 (lm % 4) is logical chunk 2 dt + (lm % 4) / 2, byte 8 (lm % 2).
+template <int CPR>
+__device__ __forceinline__ bf16x8 v_operand(const char* vb, int dt, int g, int lm) {
+  typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
+  auto rd = [&](int h) {
+    const int row = 8 * g + 4 * h + lm / 4;
+    return row * CPR * 16 + (((2 * dt + (lm % 4) / 2) ^ swz_v<CPR>(row)) * 16) + 8 * (lm % 2);
+  };
+  const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vb + rd(0)));
+  const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vb + rd(1)));
+  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
 #ifndef CKV_ATTN_PRIO
 #define CKV_ATTN_PRIO 0  // 1: raise the wavefront's issue priority around its matrix-core sections
 #endif
 #ifndef CKV_ATTN_MFMA_SUM
 #define CKV_ATTN_MFMA_SUM 1  // softmax row sums on the matrix cores (a ones operand) instead of VALU adds
 #endif
-#ifndef CKV_ATTN_XCD
-#define CKV_ATTN_XCD 1  // place the workgroups of one KV head on the same XCDs
-#endif
 constexpr int kXcds = 8;  // MI355X: workgroups go round-robin to 8 XCDs, each with its own L2
 
-// Work item (query block qb, query head hq, cache split z) of this workgroup. The hardware hands
-// workgroup L (x fastest, then y, then z) to XCD L % 8, so items are assigned through L: the
-// XCDs split evenly over the KV heads (8 / Hkv XCDs each), every item of one KV head lands on
-// that head's XCDs (its K/V stay in their L2s and are read there by all `group` query heads
-// together), consecutive items of an XCD cycle through the group's query heads on one query
-// block and split, and query blocks go latest position first, alternating between the head's
-// XCDs so their work stays balanced. Items that do not fill a last round of 8 are dealt to the
-// workgroups of that round. A bijection of the grid; with a KV-head count that does not divide 8
-// the plain order is kept.
-__device__ __forceinline__ void attn_work_item(int nqb, int Hq, int group, int& qb, int& hq, int& z) {
-  qb = nqb - 1 - (int)blockIdx.x;  // latest positions (most keys) first
-  hq = (int)blockIdx.y;
-  z = (int)blockIdx.z;
-  const int Hkv = Hq / group;
-  if (!CKV_ATTN_XCD || kXcds % Hkv != 0) return;
-  const int L = (int)blockIdx.x + ((int)blockIdx.y + (int)blockIdx.z * Hq) * nqb;
-  const int xpk = kXcds / Hkv, P = group * nqb * (int)gridDim.z;  // XCDs, items per KV head
-  const int per = P * Hkv / kXcds, full = per * kXcds;              // complete rounds of 8 workgroups
-  int kv, j;
-  if (L < full) {
-    const int xcd = L % kXcds, idx = L / kXcds;
-    kv = xcd / xpk;
-    j = idx * xpk + xcd % xpk;
-  } else {
-    const int left = P - xpk * per;  // items per KV head past the complete rounds (> 0 here)
-    const int t = L - full;
-    kv = t / left;
-    j = xpk * per + t % left;
-  }
-  const int rest = j / group;
-  hq = kv * group + j % group;
-  qb = nqb - 1 - rest % nqb;
-  z = rest / nqb;
+// Which work item (query block qb, head h, cache split z) a workgroup takes. The hardware hands
+// workgroup L of a 1-D grid to XCD L % 8, so items are assigned through L: the XCDs split evenly
+// over the KV heads (8 / Hkv XCDs each), every item of one KV head lands on that head's XCDs (its
+// K/V stay in their L2s and are read there by all `group` query heads together), consecutive items
+// of an XCD cycle through the group's query heads on one query block and split, and query blocks
+// go latest position first, alternating between the head's XCDs so their work stays balanced. The
+// grid is padded to whole rounds of 8; a workgroup past a head's last item returns. With a KV-head
+// count that does not divide 8, all heads are one group over all XCDs. The two divisions are
+// multiplications by the host's reciprocals: hardware has no integer division, and four or five
+// emulated ones were half a microsecond of every workgroup's start.
+struct AttnMap {
+  int nqb = 0, group = 0, xpk_log = 0, items = 0;  // items: of one KV head
+  uint32_t inv_group = 0, inv_nqb = 0;
+  dim3 grid;
+};
+
+// x / d for d > 0: through inv = ceil(2^32 / d) where the host found that exact for every x here
+// (x d < 2^32), 0 elsewhere.
+__device__ __forceinline__ int div_by(int x, int d, uint32_t inv) {
+  return inv != 0 ? (int)__umulhi((uint32_t)x, inv) : d == 1 ? x : x / d;
+}
+static uint32_t inverse_of(int64_t most, int64_t d) {  // for x <= most
+  return d > 1 && most * d < (1ll << 32) ? (uint32_t)(((1ll << 32) + d - 1) / d) : 0;
 }
 
-// GROUPED (few queries, decode): a workgroup's query rows are (token, query head) pairs of ONE KV
-// head, row r = token r / group, head hk * group + r % group, so the group's query heads share
-// every K/V tile the workgroup loads (grid y = KV heads); otherwise rows are tokens of one query
-// head (grid y = query heads).
-template <int D, bool GROUPED>
+__device__ __forceinline__ bool attn_work_item(int nqb, int group, int xpk_log, int items, uint32_t inv_group,
+                                               uint32_t inv_nqb, int& qb, int& h, int& z) {
+  const int L = (int)blockIdx.x, xcd = L % kXcds;
+  const int j = ((L / kXcds) << xpk_log) + (xcd & ((1 << xpk_log) - 1));
+  const int rest = div_by(j, group, inv_group);
+  h = (xcd >> xpk_log) * group + (j - rest * group);
+  z = div_by(rest, nqb, inv_nqb);
+  qb = nqb - 1 - (rest - z * nqb);
+  return j < items;
+}
+
+static AttnMap attn_map(int64_t nqb, int Hkv, int group, int64_t splits) {
+  AttnMap m;
+  if (kXcds % Hkv != 0) {
+    group *= Hkv;
+    Hkv = 1;
+  }
+  while ((Hkv << m.xpk_log) < kXcds) ++m.xpk_log;
+  m.nqb = (int)nqb;
+  m.group = group;
+  m.items = (int)(group * nqb * splits);
+  m.inv_group = inverse_of(m.items, group);
+  m.inv_nqb = inverse_of(nqb * splits, nqb);
+  m.grid = dim3((unsigned)((((int64_t)m.items + (1 << m.xpk_log) - 1) >> m.xpk_log) * kXcds));
+  return m;
+}
+
+template <int D>
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
-    char* __restrict__ out, const char* __restrict__ q, int64_t q_hs_b, int64_t q_ts_b,
-    const char* __restrict__ kc, const char* __restrict__ vc, int64_t kv_hs_b,
-    const int64_t* __restrict__ pos, int n, int N, int Hq, int group, float scale_log2, int split_tiles,
-    float* __restrict__ ws, int32_t* __restrict__ err) {
+    int nqb, int map_group, int xpk_log, int items, uint32_t inv_group, uint32_t inv_nqb,
+    const int64_t* __restrict__ pos, int n, int N, const char* __restrict__ kc, const char* __restrict__ vc,
+    int64_t kv_hs_b, const char* __restrict__ q, int64_t q_hs_b, int64_t q_ts_b, int Hq, int group, float scale_log2,
+    char* __restrict__ out, int32_t* __restrict__ err) {
   constexpr int DS = D / 32;          // k-steps of S^T = K Q^T
   constexpr int DT = D / 16;          // 16-row tiles of O^T
   constexpr int CPR = D / 8;          // 16-byte chunks per cache row
@@ -154,32 +182,16 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
   const int g = lane / 16, lm = lane % 16;
   int qb, hq, z;
-  if (GROUPED) {
-    int hk0;
-    attn_work_item((int)gridDim.x, Hq / group, 1, qb, hk0, z);
-    hq = hk0 * group;  // the group's first query head
-  } else {
-    attn_work_item((int)gridDim.x, Hq, group, qb, hq, z);
-  }
+  if (!attn_work_item(nqb, map_group, xpk_log, items, inv_group, inv_nqb, qb, hq, z)) return;
   const int hk = hq / group;
   const int q0 = qb * kAttnBM + wave * kAttnQG * 16;
-  const int n_rows = GROUPED ? n * group : n;
-  // This lane's query rows: token row_m and query head row_h (row_m >= n: no query).
-  int row_m[kAttnQG], row_h[kAttnQG];
-#pragma unroll
-  for (int qg = 0; qg < kAttnQG; ++qg) {
-    const int r = q0 + qg * 16 + lm;
-    row_m[qg] = r < n_rows ? (GROUPED ? r / group : r) : n;
-    row_h[qg] = GROUPED ? hq + r % group : hq;
-  }
-
   // Positions of this lane's queries (-1 = no query); out-of-range positions are flagged and
   // clamped so that every read stays inside the cache.
   int my_pos[kAttnQG];
   int wmax = -1, wmin = N;
 #pragma unroll
   for (int qg = 0; qg < kAttnQG; ++qg) {
-    const int m = row_m[qg];
+    const int m = q0 + qg * 16 + lm;
     int p = -1;
     if (m < n) {
       const int64_t p64 = pos[m];
@@ -204,21 +216,17 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   int bmax = blk_max_s[0];
 #pragma unroll
   for (int w = 1; w < kAttnWaves; ++w) bmax = max(bmax, blk_max_s[w]);
-  // This workgroup's share of the cache tiles: all of them, or split z of the key range when the
-  // launch is split (flash-decoding: few queries, long cache) and partials go to ws.
-  const int all_tiles = bmax < 0 ? 0 : bmax / kAttnBN + 1;
-  const int tile_begin = ws != nullptr ? z * split_tiles : 0;
-  const int n_tiles = ws != nullptr ? min(all_tiles, tile_begin + split_tiles) : all_tiles;
+  const int n_tiles = bmax < 0 ? 0 : bmax / kAttnBN + 1;
 
   // Q fragments (B operand of S^T): query q0 + 16 qg + lm, head-dim 32 s + 8 g .. + 8.
   bf16x8 qf[kAttnQG][DS];
 #pragma unroll
   for (int qg = 0; qg < kAttnQG; ++qg) {
-    const int m = row_m[qg];
+    const int m = q0 + qg * 16 + lm;
 #pragma unroll
     for (int s = 0; s < DS; ++s) {
       vec16 v = {0, 0, 0, 0};
-      if (m < n) v = ld16(q + (int64_t)row_h[qg] * q_hs_b + (int64_t)m * q_ts_b + (32 * s + 8 * g) * 2);
+      if (m < n) v = ld16(q + (int64_t)hq * q_hs_b + (int64_t)m * q_ts_b + (32 * s + 8 * g) * 2);
       qf[qg][s] = __builtin_bit_cast(bf16x8, v);
     }
   }
@@ -276,17 +284,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   int k_rd[DS];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) k_rd[ds] = lm * ROWB + (((4 * ds + g) ^ swz_k<CPR>(lm)) * 16);
-  // O^T's A operand (V^T rows) comes from row-major V through transposing 64-bit LDS loads:
-  // in each 16-lane group, lane m names row 4h + m / 4 (of the group's 8 keys 8 g ..) at column
-  // 4 (m % 4) of the 16-column tile, and lane 4a + b receives column 4a + b of rows 4h + 0..3.
-  // So lane (g, lm) holds V[8 g + 4 h + e][16 dt + lm], e = 0..3: two loads (h = 0, 1) give the
-  // eight keys 8 g + e' the B operand (P^T) pairs with that lane. Element 16 dt + 4 (lm % 4) is
-  // logical chunk 2 dt + (lm % 4) / 2, byte 8 (lm % 2).
-  auto v_rd = [&](int h, int dt) {
-    const int row = 8 * g + 4 * h + lm / 4;
-    return row * ROWB + (((2 * dt + (lm % 4) / 2) ^ swz_v<CPR>(row)) * 16) + 8 * (lm % 2);
-  };
-  if (tile_begin < n_tiles) issue(tile_begin * kAttnBN, k_lds0, v_lds0);
+  if (n_tiles > 0) issue(0, k_lds0, v_lds0);
 
   // One tile; the loop below alternates the buffers (each call names its buffers directly, so
   // the compiler sees that the loads in flight never alias the buffer being read).
@@ -379,11 +377,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
-        const char* vb = v_lds + kb * 32 * ROWB;
-        const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vb + v_rd(0, dt)));
-        const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16*)(vb + v_rd(1, dt)));
-        const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        const bf16x8 a = v_operand<CPR>(v_lds + kb * 32 * ROWB, dt, g, lm);
 #pragma unroll
         for (int qg = 0; qg < kAttnQG; ++qg)
           o[qg][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[qg][kb], o[qg][dt], 0, 0, 0);
@@ -395,32 +389,19 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
       }
     if (CKV_ATTN_PRIO) __builtin_amdgcn_s_setprio(0);
   };
-  for (int tile = tile_begin; tile < n_tiles; tile += 2) {
+  for (int tile = 0; tile < n_tiles; tile += 2) {
     body(tile, k_lds0, v_lds0, k_lds1, v_lds1);
     if (tile + 1 < n_tiles) body(tile + 1, k_lds1, v_lds1, k_lds0, v_lds0);
   }
 
   // Normalise and write: lane (g, lm) holds O[query][dt*16 + 4g + e], 4 bf16 = 8 bytes per tile.
-  // A split launch writes the unnormalised fp32 rows with their (max, sum) instead; the combine
-  // kernel merges the splits.
 #pragma unroll
   for (int qg = 0; qg < kAttnQG; ++qg) {
     const float l = CKV_ATTN_MFMA_SUM ? l_acc[qg][0] : group_sum(l_run[qg]);
-    const int m = row_m[qg], h = row_h[qg];
+    const int m = q0 + qg * 16 + lm;
     if (m >= n) continue;
-    if (ws != nullptr) {
-      float* prow = ws + (((int64_t)z * Hq + h) * n + m) * (D + 4);  // 16-byte aligned rows
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) *(float4*)(prow + dt * 16 + 4 * g) = make_float4(o[qg][dt][0], o[qg][dt][1],
-                                                                                    o[qg][dt][2], o[qg][dt][3]);
-      if (g == 0) {
-        prow[D] = m_run[qg];
-        prow[D + 1] = l;
-      }
-      continue;
-    }
     const float inv = 1.f / l;
-    char* orow = out + ((int64_t)m * Hq + h) * (D * 2);
+    char* orow = out + ((int64_t)m * Hq + hq) * (D * 2);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       unsigned w[2];
@@ -431,114 +412,85 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   }
 }
 
-// Merge the splits of a split launch: for query m and head h, with (M_z, L_z, O_z) the partials
-// of split z (max in the log2 domain, sum and unnormalised rows relative to M_z):
-//   out = sum_z 2^(M_z - M) O_z / sum_z 2^(M_z - M) L_z,  M = max_z M_z  (splits with M_z = -inf
-// saw no visible row and weigh 0). One workgroup of kCombineWaves wavefronts per (query, head):
-// wavefront w folds splits w*4 .. w*4+3, then every (4 x kCombineWaves)-th group after them,
-// loading each group's four partials together and merging them into a running (max, sum, row)
-// with the online rescale; the wavefronts' results are merged through LDS. Lane d covers
-// head-dim columns d, d + 64.
-constexpr int kCombineWaves = 4;
-
-template <int D>
-__global__ __launch_bounds__(kCombineWaves * 64) void attn_combine_kernel(char* __restrict__ out,
-                                                                          const float* __restrict__ ws, int n, int Hq,
-                                                                          int splits) {
-  constexpr int CW = D / 64;  // columns per lane
-  constexpr int U = 4;        // partials in flight per wavefront
-  const int m = blockIdx.x, hq = blockIdx.y, lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int64_t stride = (int64_t)Hq * n * (D + 4);
-  const float* base = ws + ((int64_t)hq * n + m) * (D + 4);
-  float M = -INFINITY, L = 0.f, acc[CW];
-#pragma unroll
-  for (int j = 0; j < CW; ++j) acc[j] = 0.f;
-  for (int z0 = wave * U; z0 < splits; z0 += U * kCombineWaves) {
-    float mz[U], lz[U], oz[U][CW];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      mz[u] = -INFINITY;
-      lz[u] = 0.f;
-#pragma unroll
-      for (int j = 0; j < CW; ++j) oz[u][j] = 0.f;
-      if (z0 + u < splits) {
-        const float* pz = base + (int64_t)(z0 + u) * stride;
-        mz[u] = pz[D];
-        lz[u] = pz[D + 1];
-#pragma unroll
-        for (int j = 0; j < CW; ++j) oz[u][j] = pz[lane + 64 * j];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (mz[u] == -INFINITY) continue;  // uniform: the same partial for every lane
-      const float mn = fmaxf(M, mz[u]);
-      const float a = __builtin_amdgcn_exp2f(M - mn);  // 0 while M is still -inf
-      const float b = __builtin_amdgcn_exp2f(mz[u] - mn);
-      L = L * a + lz[u] * b;
-#pragma unroll
-      for (int j = 0; j < CW; ++j) acc[j] = acc[j] * a + oz[u][j] * b;
-      M = mn;
-    }
-  }
-  __shared__ float s_m[kCombineWaves], s_l[kCombineWaves], s_o[kCombineWaves][D];
-  if (lane == 0) {
-    s_m[wave] = M;
-    s_l[wave] = L;
-  }
-#pragma unroll
-  for (int j = 0; j < CW; ++j) s_o[wave][lane + 64 * j] = acc[j];
-  __syncthreads();
-  if (wave != 0) return;
-  float mx = -INFINITY;
-#pragma unroll
-  for (int w = 0; w < kCombineWaves; ++w) mx = fmaxf(mx, s_m[w]);
-  float lt = 0.f, o[CW];
-#pragma unroll
-  for (int j = 0; j < CW; ++j) o[j] = 0.f;
-#pragma unroll
-  for (int w = 0; w < kCombineWaves; ++w) {
-    if (s_m[w] == -INFINITY) continue;
-    const float sw = __builtin_amdgcn_exp2f(s_m[w] - mx);
-    lt += sw * s_l[w];
-#pragma unroll
-    for (int j = 0; j < CW; ++j) o[j] += sw * s_o[w][lane + 64 * j];
-  }
-  const float inv = 1.f / lt;
-  uint16_t* orow = reinterpret_cast<uint16_t*>(out + ((int64_t)m * Hq + hq) * (D * 2));
-#pragma unroll
-  for (int j = 0; j < CW; ++j) orow[lane + 64 * j] = (uint16_t)f32_to_bf16_bits(o[j] * inv);
-}
-
 }  // namespace ckv
+
+#include "attention_wave.hpp"
 
 namespace ckv {
 
-#ifndef CKV_ATTN_GSPLIT
-#define CKV_ATTN_GSPLIT 3
-#endif
-constexpr int kGroupedSplitTiles = CKV_ATTN_GSPLIT;  // cache tiles per split of a grouped launch
+// How a launch runs.
+struct AttnPlan {
+  bool wave = false;     // attn_wave_kernel, else attn_active_kernel
+  bool grouped = false;  // rows are the (token, query head) pairs of a KV head
+  int qg = 0, waves = 0;
+  int splits = 1, split_chunks = 0;
+  AttnMap map;
+};
 
-// Split plan of a launch whose rows are tokens of one query head: split only launches too small
-// to fill the chip (decode-like), into about 1024 workgroups of >= 4 tiles each.
-static void row_split_plan(int n_queries, int n_tokens, int n_q_heads, int& splits, int& split_tiles) {
-  splits = 1;
-  split_tiles = 0;
-  const int64_t blocks = (int64_t)((n_queries + kAttnBM - 1) / kAttnBM) * n_q_heads;
-  const int tiles = (n_tokens + kAttnBN - 1) / kAttnBN;
-  constexpr int64_t kTarget = 1024;  // workgroups that fill the 256 CUs a few times over
-  if (blocks < kTarget / 2 && tiles >= 8) {
-    const int want = (int)std::min<int64_t>((kTarget + blocks - 1) / blocks, tiles / 4);
-    split_tiles = (tiles + want - 1) / want;
-    splits = (tiles + split_tiles - 1) / split_tiles;
-  }
+// The (head_dim, QG, W, GROUPED) forms of attn_wave_kernel that attn_plan picks from.
+#define CKV_WAVE_FORMS(X)                                                                  \
+  X(128, 1, 4, true) X(128, 1, 8, true) X(128, 2, 8, true)                                  \
+  X(128, 1, 4, false) X(128, 1, 8, false) X(128, 2, 4, false) X(128, 2, 8, false)           \
+  X(64, 1, 4, true) X(64, 1, 8, true)                                                       \
+  X(64, 1, 4, false) X(64, 1, 8, false) X(64, 2, 4, false) X(64, 2, 8, false)
+
+// Where the 128-query workgroups are too few: below about one for each of the 256 CUs at head_dim
+// 128 (us, 28 heads: 1103 causal rows, 252 workgroups, 27.7 against 29.5; 2000 rows, 448, 63.7
+// against 51.1), below two at head_dim 64, where they also hold less work each (14 heads: 4000
+// rows, 448 workgroups, 57.3 against 69.0; 6000, 658, 119 against 105).
+static bool wave_launch(int n, int Hq, int head_dim) {
+  const int64_t blocks = (int64_t)((n + kAttnBM - 1) / kAttnBM) * Hq;
+  return blocks < (head_dim == 128 ? 256 : 512);
 }
 
-// Grouped launches (queries that share KV heads fit one workgroup's rows): every
-// kGroupedSplitTiles cache tiles are one split. Usable when n_queries * group <= kAttnBM.
-static void grouped_split_plan(int n_queries, int n_tokens, int& splits) {
-  const int tiles = (n_tokens + kAttnBN - 1) / kAttnBN;
-  splits = (2 * n_queries <= kAttnBM && tiles >= 2) ? (tiles + kGroupedSplitTiles - 1) / kGroupedSplitTiles : 1;
+constexpr int kWaveFill = 256;  // workgroups that a split launch aims at: one for each CU
+
+// The most splits a launch takes: a workgroup has at most 32 (token, query head) rows, a split's
+// four wavefronts a chunk each.
+static int64_t most_splits(int n, int N, int Hq, int head_dim) {
+  const int64_t chunks = (N + kWaveChunk - 1) / kWaveChunk;
+  if (!wave_launch(n, Hq, head_dim) || chunks <= 16) return 1;
+  return std::max<int64_t>(1, std::min<int64_t>(kWaveFill * 32 / ((int64_t)n * Hq), (chunks + 3) / 4));
+}
+
+static AttnPlan attn_plan(int n, int N, int Hq, int Hkv, int head_dim, int64_t workspace_bytes) {
+  AttnPlan p;
+  const int group = Hq / Hkv;
+  if (!wave_launch(n, Hq, head_dim)) {
+    p.map = attn_map((n + kAttnBM - 1) / kAttnBM, Hkv, group, 1);
+    return p;
+  }
+  p.wave = true;
+  p.grouped = group > 1 && (int64_t)n * group <= kAttnBM;
+  const int rows = p.grouped ? n * group : n, heads = p.grouped ? Hkv : Hq;
+  const int chunks = (N + kWaveChunk - 1) / kWaveChunk;
+  const int b16 = (rows + 15) / 16 * heads, b32 = (rows + 31) / 32 * heads;
+  // 16 rows a workgroup while those workgroups are all resident at once (two or four of four
+  // wavefronts on a CU, by registers), else 32, which read each cache row half as often: 28 heads
+  // of 128, 192 causal rows 5.9 against 7.2 us, 320 rows (560 workgroups) 9.8 against 9.0. A long
+  // cache is read often enough to prefer 32 earlier at head_dim 128 (251 of 1103 rows 13.7 against
+  // 14.1, 300 of 4000 34 against 43).
+  const bool lng = chunks >= 24;
+  if (rows <= 16) p.qg = 1;
+  else if (lng) p.qg = head_dim == 64 && b16 <= 512 ? 1 : 2;
+  else p.qg = b16 <= (head_dim == 64 ? 800 : 512) ? 1 : 2;
+  const int blocks = p.qg == 1 ? b16 : b32;
+  // Eight wavefronts halve a workgroup's chain where it is long, if the workgroups still fit (one
+  // or two on a CU): 300 of 4000 rows 34 against 45 us with four, 768 causal rows 24.5 against 19.1.
+  p.waves = lng && (blocks <= 288 || (blocks <= 450 && chunks >= 128)) ? 8 : 4;
+  // Splits cost the merge launch, about 3 us: taken for one token's rows from 17 chunks on (28
+  // heads, 700 rows 7.1 against 8.5 us, 8288 rows 8.7 against 45), else where eight wavefronts
+  // would have eight chunks each (150 of 1500 rows, 47 chunks, 8.5 us whole and 9.5 in two).
+  int64_t splits = std::min<int64_t>(most_splits(n, N, Hq, head_dim), kWaveFill / std::max(blocks, 1));
+  if (rows > 16 && chunks < 64) splits = 1;
+  const int64_t row_b = (int64_t)Hq * n * (head_dim + 4) * 4;
+  splits = std::min<int64_t>(splits, workspace_bytes / row_b);
+  if (rows <= 16) p.waves = splits > 1 ? 4 : 8;
+  splits = std::max<int64_t>(1, std::min<int64_t>(splits, (chunks + p.waves - 1) / p.waves));
+  p.split_chunks = (int)((chunks + splits - 1) / splits);
+  p.splits = (chunks + p.split_chunks - 1) / p.split_chunks;
+  p.map = attn_map(blocks / heads, Hkv, p.grouped ? 1 : group, p.splits);
+  return p;
 }
 
 }  // namespace ckv
@@ -546,16 +498,13 @@ static void grouped_split_plan(int n_queries, int n_tokens, int& splits) {
 extern "C" int64_t ckv_attention_workspace_bytes(int32_t n_queries, int32_t n_tokens, int32_t n_q_heads,
                                                  int32_t head_dim, int32_t* splits_out, int32_t* split_tiles_out) {
   using namespace ckv;
-  int splits = 1, split_tiles = 0, gsplits = 1;
-  if (n_queries > 0 && n_tokens > 0 && n_q_heads > 0 && head_dim > 0) {
-    row_split_plan(n_queries, n_tokens, n_q_heads, splits, split_tiles);
-    grouped_split_plan(n_queries, n_tokens, gsplits);
-  }
-  if (splits_out != nullptr) *splits_out = splits;
-  if (split_tiles_out != nullptr) *split_tiles_out = split_tiles;
-  const int64_t row = (int64_t)n_q_heads * n_queries * (head_dim + 4) * 4;
-  const int64_t most = std::max(splits > 1 ? splits : 0, gsplits > 1 ? gsplits : 0);
-  return most * row;
+  int64_t splits = 1;
+  if (n_queries > 0 && n_tokens > 0 && n_q_heads > 0 && head_dim > 0)
+    splits = most_splits(n_queries, n_tokens, n_q_heads, head_dim);
+  const int tiles = n_tokens > 0 ? (n_tokens + kAttnBN - 1) / kAttnBN : 0;
+  if (splits_out != nullptr) *splits_out = (int32_t)splits;
+  if (split_tiles_out != nullptr) *split_tiles_out = splits > 1 ? (int32_t)((tiles + splits - 1) / splits) : 0;
+  return splits > 1 ? splits * n_q_heads * n_queries * (head_dim + 4) * 4 : 0;
 }
 
 extern "C" int32_t ckv_attention_active(void* out, const void* q, int64_t q_head_stride, int64_t q_token_stride,
@@ -579,40 +528,45 @@ extern "C" int32_t ckv_attention_active(void* out, const void* q, int64_t q_head
   const float scale_log2 = (float)(scale * 1.4426950408889634);  // exp(x) = exp2(x log2 e)
   const int group = n_q_heads / n_kv_heads;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t row_b = (int64_t)n_q_heads * n_queries * (head_dim + 4) * 4;
-  const bool ws_ok = workspace != nullptr && (uintptr_t)workspace % 16 == 0;
-  auto launch = [&](auto kernel, auto combine, dim3 grid, int split_tiles, float* ws, int splits) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kAttnWaves * 64), 0, st, (char*)out, (const char*)q, q_head_stride * 2,
-                       q_token_stride * 2, (const char*)k_cache, (const char*)v_cache, kv_head_stride * 2, positions,
-                       n_queries, n_tokens, n_q_heads, group, scale_log2, split_tiles, ws, err);
-    if (ws != nullptr)
-      hipLaunchKernelGGL(combine, dim3((unsigned)n_queries, (unsigned)n_q_heads), dim3(kCombineWaves * 64), 0, st,
-                         (char*)out, ws,
-                         n_queries, n_q_heads, splits);
-  };
-  // Queries that share KV heads and fit one workgroup's rows (decode): one workgroup per
-  // (KV head, split), all of the group's query heads on each loaded K/V tile.
-  int gsplits = 1;
-  grouped_split_plan(n_queries, n_tokens, gsplits);
-  if (group > 1 && (int64_t)n_queries * group <= kAttnBM && gsplits > 1 && ws_ok &&
-      workspace_bytes >= gsplits * row_b) {
-    const dim3 grid(1u, (unsigned)n_kv_heads, (unsigned)gsplits);
-    if (head_dim == 128)
-      launch(attn_active_kernel<128, true>, attn_combine_kernel<128>, grid, kGroupedSplitTiles, (float*)workspace, gsplits);
-    else
-      launch(attn_active_kernel<64, true>, attn_combine_kernel<64>, grid, kGroupedSplitTiles, (float*)workspace, gsplits);
+  const AttnPlan plan = attn_plan(n_queries, n_tokens, n_q_heads, n_kv_heads, head_dim,
+                                  workspace != nullptr && (uintptr_t)workspace % 16 == 0 ? workspace_bytes : 0);
+  const AttnMap& map = plan.map;
+  if (!plan.wave) {
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, map.grid, dim3(kAttnWaves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
+                         map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
+                         (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
+                         n_q_heads, group, scale_log2, (char*)out, err);
+    };
+    if (head_dim == 128) launch(attn_active_kernel<128>);
+    else launch(attn_active_kernel<64>);
     CKV_RETURN_IF_LAUNCH_FAILED();
     return CKV_OK;
   }
-  int splits = 1, split_tiles = 0;
-  row_split_plan(n_queries, n_tokens, n_q_heads, splits, split_tiles);
-  float* ws = (splits > 1 && ws_ok && workspace_bytes >= splits * row_b) ? (float*)workspace : nullptr;
-  if (ws == nullptr) splits = 1;
-  const dim3 grid((unsigned)((n_queries + kAttnBM - 1) / kAttnBM), (unsigned)n_q_heads, (unsigned)splits);
-  if (head_dim == 128)
-    launch(attn_active_kernel<128, false>, attn_combine_kernel<128>, grid, split_tiles, ws, splits);
-  else
-    launch(attn_active_kernel<64, false>, attn_combine_kernel<64>, grid, split_tiles, ws, splits);
+  float* ws = plan.splits > 1 ? (float*)workspace : nullptr;
+  const uint32_t inv_gqa = inverse_of((int64_t)n_queries * group, group);
+  auto launch = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, map.grid, dim3(waves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
+                       map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
+                       (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
+                       n_q_heads, group, inv_gqa, scale_log2, plan.split_chunks, (char*)out, ws, err);
+  };
+#define CKV_WAVE(HD, QG, W, GR) \
+  else if (head_dim == HD && plan.qg == QG && plan.waves == W && plan.grouped == GR) \
+    launch(attn_wave_kernel<HD, QG, W, GR>, W);
+  if (false) {
+  }
+  CKV_WAVE_FORMS(CKV_WAVE)
+  else return CKV_ERR_INVALID_ARGUMENT;  // a plan outside the list
+#undef CKV_WAVE
   CKV_RETURN_IF_LAUNCH_FAILED();
+  if (ws != nullptr) {
+    const dim3 grid((unsigned)n_queries, (unsigned)n_q_heads);
+    const dim3 block(64 * (unsigned)std::min((plan.splits + kCombineParts - 1) / kCombineParts, kCombineMaxWaves));
+    auto merge = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, (char*)out, ws, n_queries, n_q_heads, plan.splits); };
+    if (head_dim == 128) merge(attn_combine_kernel<128>);
+    else merge(attn_combine_kernel<64>);
+    CKV_RETURN_IF_LAUNCH_FAILED();
+  }
   return CKV_OK;
 }

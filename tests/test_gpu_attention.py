@@ -116,3 +116,40 @@ def test_attention_split_launch_matches_oracle_and_unsplit(Hq, Hkv, D, N, n):
     torch.cuda.synchronize()
     torch.testing.assert_close(split.float(), whole.float(), atol=4e-3, rtol=0)
     np.testing.assert_allclose(split[0].float().cpu().numpy(), O.attention_active(q, K, V, pos), atol=ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,N,n", [
+    (28, 4, 128, 1, 1),      # one cache row
+    (28, 4, 128, 31, 31),    # less than one 32-row chunk
+    (12, 3, 64, 33, 17),     # KV heads that do not divide the 8 XCDs; one row past a chunk and past 16 rows
+    (28, 4, 128, 320, 320),  # 32 rows a workgroup (more 16-row workgroups than fit at once)
+    (14, 2, 64, 200, 200),   # 16 rows a workgroup, last one ragged
+    (28, 4, 128, 512, 2),    # one token's worth of rows over 16 chunks: not split
+    (28, 4, 128, 513, 2),    # 17 chunks: split, the last split one row long
+    (28, 4, 128, 767, 251),  # 24 chunks: eight wavefronts
+    (14, 2, 64, 1103, 251),  # eight wavefronts, 16 rows each
+    (28, 4, 64, 4100, 150),  # eight wavefronts, 16 rows, 129 chunks
+    (28, 4, 128, 1180, 1152),  # 252 128-query workgroups: the last size below the large kernel's range
+    (28, 4, 128, 1181, 1153),  # 280: the first inside it
+    (16, 16, 64, 2100, 40),  # no grouping, split
+])
+def test_attention_small_launch_forms(Hq, Hkv, D, N, n):
+    """Every form of the small-launch kernel (rows and wavefronts per workgroup, grouped rows, splits)
+    at the edges of its range: against the oracle, unsplit, and with the rows past every position
+    uninitialised (NaN), which no query may see. Tolerance as at the top of this file."""
+    q, K, V, pos = _case(N * 7 + n, Hq, Hkv, D, N, n)
+    seen = max(1, N - 3)
+    pos = np.minimum(pos, seen - 1)
+    K[:, seen:], V[:, seen:] = 0x7FC0, 0x7FC0
+    args = [O.from_numpy(a, DEV)[None] for a in (q, K, V)] + [torch.from_numpy(pos).to(DEV)]
+    got = ops.attention_active(*args)
+    whole = ops.attention_active(*args, split=False)
+    sub = np.unique(np.linspace(0, n - 1, min(n, 200)).astype(int))
+    want = O.attention_active(q[:, sub], K[:, :seen], V[:, :seen], pos[sub])
+    small = -(-n // 128) * Hq < (256 if D == 128 else 512)
+    for out in (got, whole) if small else ():
+        np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
+    if not small:  # the large kernel multiplies zero weights into the rest of its last tile
+        K[:, seen:], V[:, seen:] = 0, 0
+        out, _ = _run(q, K, V, pos)
+        np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
