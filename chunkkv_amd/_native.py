@@ -8,12 +8,15 @@ valid inside the library. There is no fallback: if the library is missing, every
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from pathlib import Path
 
 import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libchunkkv_amd.so"
+TORCH_OPS_PATH = LIB_PATH.with_name("_torch_ops.so")
 ABI_VERSION = 5
 
 CKV_OK = 0
@@ -152,6 +155,23 @@ def lib() -> ctypes.CDLL:
             raise NativeLibraryMissing(f"{LIB_PATH} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")
         _lib = handle
     return _lib
+
+
+_ops = None
+
+
+def torch_ops():
+    """The native per-layer calls (csrc/torch_ops.cpp); raises NativeLibraryMissing if not built."""
+    global _ops
+    if _ops is None:
+        lib()  # the library they call, and its ABI version
+        if not TORCH_OPS_PATH.exists():
+            raise NativeLibraryMissing(f"{TORCH_OPS_PATH} is not built; run `python -m chunkkv_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("_torch_ops", str(TORCH_OPS_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_torch_ops", loader))
+        loader.exec_module(module)
+        _ops = module
+    return _ops
 
 
 def check(status: int, what: str) -> None:

@@ -2,7 +2,8 @@
 
 Run ``python -m chunkkv_amd.build``. hipcc cross-compiles for gfx950 without a GPU. The
 library is a plain C-ABI shared object (see ``include/chunkkv_amd.h``); Python loads it with
-ctypes after ``import torch`` so that it binds to the HIP runtime torch already loaded.
+ctypes after ``import torch`` so that it binds to the HIP runtime torch already loaded. The
+per-layer calls (``csrc/torch_ops.cpp``) are a CPython module beside it, built against torch.
 """
 
 from __future__ import annotations
@@ -11,6 +12,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -22,6 +24,7 @@ LIB_NAME = "libchunkkv_amd.so"
 SOURCES = ["abi.hip", "rerope_gather.hip", "assemble.hip", "deviation.hip", "select.hip", "select_gather.hip", "deviation_select.hip",
            "scatter.hip", "layer1_repair.hip", "attention.hip", "rope.hip", "extract.hip", "norm.hip"]
 HOST_SOURCES = ["token_hash.cpp"]
+TORCH_SOURCE, TORCH_OPS_NAME = "torch_ops.cpp", "_torch_ops.so"
 ARCH = "gfx950"
 GXX_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-pthread", "-Wall", "-Wextra"]
 
@@ -78,7 +81,25 @@ def build(verbose: bool = False) -> Path:
     tmp = out.with_suffix(".so.tmp")
     _run([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-pthread", "-o", str(tmp)], verbose)
     os.replace(tmp, out)
+    _build_torch_ops(verbose)
     return out
+
+
+def _build_torch_ops(verbose: bool) -> None:
+    """The CPython module of the per-layer calls: host C++ against torch's headers and the library."""
+    import torch
+
+    t = Path(torch.__file__).resolve().parent
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    out = LIB_DIR / TORCH_OPS_NAME
+    tmp = out.with_suffix(".so.tmp")
+    _run(["g++", *GXX_FLAGS, "-Wno-unused-parameter", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+          "-isystem", str(t / "include"), "-isystem", str(t / "include/torch/csrc/api/include"),
+          "-isystem", f"{rocm}/include", "-isystem", sysconfig.get_paths()["include"], str(CSRC / TORCH_SOURCE),
+          "-o", str(tmp), f"-L{t / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip",
+          f"-L{LIB_DIR}", f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN"], verbose)
+    os.replace(tmp, out)
 
 
 def _run(cmd: list[str], verbose: bool) -> None:

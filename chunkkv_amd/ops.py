@@ -2,12 +2,13 @@
 
 Each wrapper checks shapes, dtypes, devices and 16-byte alignment on the host, passes raw
 device pointers and torch's current HIP stream, and maps a non-zero status to an exception.
-Every wrapper launches a HIP kernel; none computes anything on the CPU.
+Every wrapper launches a HIP kernel; none computes anything on the CPU. The calls that a request
+makes for every layer, and the two that allocate many outputs, do this in one native call
+(csrc/torch_ops.cpp).
 """
 
 from __future__ import annotations
 
-import math
 from dataclasses import dataclass
 
 import torch
@@ -476,28 +477,12 @@ def layer1_repair_gather(
     layer1_repair_gather_whole_layers(...) layers of the range (gathered whole beside the
     selection) and untouched in the others. The caller overwrites the kept rows of every gathered
     layer with that layer's fresh rows, which makes both forms the same cache. Three launches."""
-    if k_slab.dim() != 5 or v_slab.shape != k_slab.shape or not (k_slab.is_contiguous() and v_slab.is_contiguous()):
-        raise ValueError("k_slab/v_slab must be contiguous (L, 1, H, N, D)")
-    L, _, H, N, D = k_slab.shape
-    b, e = int(layers[0]), int(layers[1])
-    if not (0 <= b <= e <= L) or b <= int(layer) < e:
-        raise ValueError(f"gather layers {layers} must lie in [0, {L}) and exclude layer {layer}")
-    K, V = k_slab[int(layer)], v_slab[int(layer)]
-    k, v, diff, norm, out, C, n_tab = _layer1_args(K, V, src_tab, L, segments, n_segs, k, v, flags, local, spans,
-                                                   workspace, out, diff_norm)
-    has_thr = escalate_threshold is not None
-    check(
-        lib().ckv_layer1_repair_gather(
-            _ptr(k_slab), _ptr(v_slab), H * N * D, N * D, _ptr(src_tab), n_tab, L, int(layer), b, e, _ptr(segments),
-            int(n_segs), int(max_seg_tokens), _ptr(k), k.stride(1), k.stride(2), _ptr(v), v.stride(1), v.stride(2),
-            k.shape[2], _ptr(flags), _ptr(local), N, H, D, dtype_code(K.dtype), float(theta), _ptr(spans), C,
-            int(has_thr), float(escalate_threshold) if has_thr else 0.0, _ptr(diff), _ptr(norm), _ptr(out.keep_abs),
-            _ptr(out.keep_local), _ptr(out.keep_rank), _ptr(out.rel_dev), _ptr(out.escalated), _ptr(out.counts),
-            _ptr(workspace), workspace.numel() * workspace.element_size(), _ptr(err), _stream(K.device),
-        ),
-        "ckv_layer1_repair_gather",
-    )
-    return diff, norm, out
+    given = None if out is None else (out.keep_abs, out.keep_local, out.keep_rank, out.rel_dev, out.escalated, out.counts)
+    diff, norm, *sel = _native.torch_ops().layer1_repair_gather(
+        k_slab, v_slab, src_tab, int(layer), int(layers[0]), int(layers[1]), segments, int(n_segs), int(max_seg_tokens),
+        k, v, flags, local, spans, escalate_threshold, theta, workspace, err, given,
+        None if diff_norm is None else tuple(diff_norm))
+    return diff, norm, Selection(*sel) if out is None else out
 
 
 def layer1_repair_gather_whole_layers(n_tokens: int, n_chunks: int, escalate_threshold: float | None, n_segs: int,
@@ -644,45 +629,7 @@ def attention_active(
     split: let launches too small to fill the chip split the cache range (a workspace is
     allocated for the partial results).
     """
-    _dev(q, K, V, positions)
-    _, Hq, n, D = q.shape
-    _, Hkv, N, _ = K.shape
-    if q.dtype != torch.bfloat16 or K.dtype != torch.bfloat16 or V.dtype != torch.bfloat16:
-        raise TypeError("attention_active runs on bf16 q/K/V")
-    if not (K.is_contiguous() and V.is_contiguous() and V.shape == K.shape) or K.shape[3] != D:
-        raise ValueError("K/V must be contiguous (1, Hkv, N, D) and match q's head_dim")
-    if q.stride(3) != 1:
-        q = q.contiguous()
-    if positions.dtype != torch.int64 or positions.numel() != n:
-        raise ValueError("positions must be int64 (n,)")
-    positions = positions.contiguous()
-    if out is None:
-        out = torch.empty((1, n, Hq, D), dtype=q.dtype, device=q.device)
-    elif out.shape != (1, n, Hq, D) or not out.is_contiguous() or out.dtype != q.dtype:
-        raise ValueError("out must be contiguous (1, n, Hq, D) bf16")
-    scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    ws_bytes = lib().ckv_attention_workspace_bytes(n, N, Hq, D, None, None) if split else 0
-    ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device) if ws_bytes > 0 else None
-    check(
-        lib().ckv_attention_active(
-            _ptr(out), _ptr(q), q.stride(1), q.stride(2), _ptr(K), _ptr(V), N * D, _ptr(positions), n, N, Hq, Hkv,
-            D, dtype_code(q.dtype), scale, _ptr(ws), ws_bytes, _ptr(err), _stream(q.device),
-        ),
-        "ckv_attention_active",
-    )
-    return out
-
-
-def _heads_view(t: torch.Tensor, n_heads: int, head_dim: int) -> tuple:
-    """(pointer, head stride, token stride) of a (1, n, n_heads*D)-like token-major tensor or a
-    (1, H, n, D) tensor with contiguous rows."""
-    if t.dim() == 3:
-        if t.stride(2) != 1 or t.shape[2] != n_heads * head_dim:
-            raise ValueError("projection output must have contiguous rows of n_heads * head_dim")
-        return _ptr(t), head_dim, t.stride(1)
-    if t.dim() == 4 and t.shape[1] == n_heads and t.shape[3] == head_dim and t.stride(3) == 1:
-        return _ptr(t), t.stride(1), t.stride(2)
-    raise ValueError(f"unsupported layout {tuple(t.shape)} / {t.stride()}")
+    return _native.torch_ops().attention_active(q, K, V, positions, scale, err, out, split)
 
 
 def rope_qkv(
@@ -711,56 +658,8 @@ def rope_qkv(
     table: optional rope_table() covering every position (the same results). Without one (the
     default, and what HipEngine does) the kernel evaluates cos/sin from theta and the positions.
     """
-    if table is not None:
-        _dev(k_in, table)
-        if table.dtype != torch.float32 or table.dim() != 3 or table.shape[1:] != (head_dim // 2, 2):
-            raise ValueError("table must be a rope_table() output (n, D/2, 2) float32")
-    _dev(k_in, positions)
-    n = positions.numel()
-    dev = k_in.device
-    if n_q_heads == 0:  # k/v only
-        q_in = k_in
-    if positions.dtype != torch.int64:
-        raise ValueError("positions must be int64")
-    positions = positions.contiguous()
-    if q_out is None and n_q_heads:
-        q_out = torch.empty((1, n, n_q_heads, head_dim), dtype=q_in.dtype, device=dev)
-    if k_out is None:
-        if rows is not None:
-            raise ValueError("rows needs k_out (the cache)")
-        k_out = torch.empty((1, n_kv_heads, n, head_dim), dtype=q_in.dtype, device=dev)
-    n_out = k_out.shape[2] if k_out.dim() == 4 else k_out.shape[1]
-    if rows is not None:
-        _dev(q_in, rows)
-        if rows.dtype != torch.int64 or rows.numel() != n:
-            raise ValueError("rows must be int64 (n,)")
-        rows = rows.contiguous()
-    if (v_in is None) != (v_out is None):
-        raise ValueError("v_in and v_out go together")
-    for t in (q_in, k_in, k_out) + ((q_out,) if n_q_heads else ()) + ((v_in, v_out) if v_in is not None else ()):
-        if t.dtype != q_in.dtype:
-            raise TypeError("q/k/v and outputs must share a dtype")
-    if n_q_heads:
-        if q_out.shape != (1, n, n_q_heads, head_dim) or not q_out.is_contiguous():
-            raise ValueError("q_out must be contiguous (1, n, Hq, D), token-major")
-        qo = _heads_view(q_out.view(1, n, n_q_heads * head_dim), n_q_heads, head_dim)
-        qi = _heads_view(q_in, n_q_heads, head_dim)
-    else:
-        qo = qi = (None, 0, 0)
-    ki = _heads_view(k_in, n_kv_heads, head_dim)
-    ko = _heads_view(k_out, n_kv_heads, head_dim)
-    vi = _heads_view(v_in, n_kv_heads, head_dim) if v_in is not None else (None, 0, 0)
-    vo = _heads_view(v_out, n_kv_heads, head_dim) if v_out is not None else (None, 0, 0)
-    check(
-        lib().ckv_rope_qkv(
-            qo[0], qo[1], qo[2], ko[0], ko[1], ko[2], vo[0], vo[1], vo[2], _ptr(rows), n_out, qi[0], qi[1], qi[2],
-            ki[0], ki[1], ki[2], vi[0], vi[1], vi[2], _ptr(positions), _ptr(table),
-            0 if table is None else table.shape[0], n, n_q_heads, n_kv_heads, head_dim,
-            dtype_code(q_in.dtype), float(theta), _ptr(err), _stream(dev),
-        ),
-        "ckv_rope_qkv",
-    )
-    return q_out, k_out
+    return _native.torch_ops().rope_qkv(q_in, k_in, v_in, positions, n_q_heads, n_kv_heads, head_dim, theta, q_out, k_out,
+                                        v_out, rows, table, err)
 
 
 def rope_table(n_positions: int, head_dim: int, theta: float, device) -> torch.Tensor:
@@ -781,47 +680,7 @@ def extract_chunks(
     k_slab/v_slab: (L, 1, H, N, D) contiguous. Returns one (2, L, 1, H, end - start, D) tensor per
     span (index 0 = keys, 1 = values), each its own allocation so a store can free it alone.
     """
-    _dev(k_slab, v_slab)
-    if not (k_slab.is_contiguous() and v_slab.is_contiguous() and k_slab.shape == v_slab.shape):
-        raise ValueError("K/V slabs must be contiguous and of equal shape")
-    L, _, H, N, D = k_slab.shape
-    dev = k_slab.device
-    bufs, meta = [], []
-    for start, end in spans:
-        start, end = int(start), int(end)
-        if not 0 <= start <= end <= N:
-            raise ValueError(f"span [{start}, {end}) outside the request of {N} tokens")
-        b = torch.empty((2, L, 1, H, end - start, D), dtype=k_slab.dtype, device=dev)
-        bufs.append(b)
-        meta.append((b.data_ptr(), start, end - start))
-    live = [(p, s, n) for p, s, n in meta if n > 0]
-    if not live:
-        return bufs
-    # descriptors: [ptr lo, ptr hi] per span, then (start, len) pairs; pinned, one async copy
-    # (torch's pinned allocator keeps the host block until the copy has run)
-    pinned = torch.empty(len(live) * 4, dtype=torch.int32, pin_memory=True)
-    host = pinned.numpy()
-    host[: 2 * len(live)].view("<u8")[:] = [p for p, _, _ in live]
-    host[2 * len(live) :] = [v for _, s, n in live for v in (s, n)]
-    d = pinned.to(dev, non_blocking=True)
-    check(
-        lib().ckv_extract_chunks(
-            _ptr(k_slab), _ptr(v_slab), H * N * D, N * D, _ptr(d), d.data_ptr() + 8 * len(live), len(live),
-            max(n for _, _, n in live), L, H, N, D, dtype_code(k_slab.dtype), _ptr(err), _stream(dev),
-        ),
-        "ckv_extract_chunks",
-    )
-    return bufs
-
-
-def _row_major(t: torch.Tensor, width: int, what: str) -> int:
-    """Row stride (elements) of a (..., width) tensor whose rows are contiguous and evenly spaced."""
-    if t.shape[-1] != width or t.stride(-1) != 1 or t.data_ptr() % 16 != 0:
-        raise ValueError(f"{what} must have contiguous, 16-byte aligned rows of {width} elements")
-    rows = t.reshape(-1, width) if t.dim() != 2 else t
-    if rows.data_ptr() != t.data_ptr() or (rows.shape[0] > 1 and rows.stride(1) != 1):
-        raise ValueError(f"{what} rows must be evenly spaced")
-    return rows.stride(0) if rows.shape[0] > 1 else width
+    return _native.torch_ops().extract_chunks(k_slab, v_slab, spans, err)
 
 
 def add_rmsnorm(
@@ -840,49 +699,11 @@ def add_rmsnorm(
     :113, :75). h, delta: (..., hidden) contiguous; h_out defaults to a new tensor and may be h
     itself (in place).
     """
-    _dev(h, weight, *(() if delta is None else (delta,)))
-    hidden = h.shape[-1]
-    if not h.is_contiguous() or (delta is not None and (not delta.is_contiguous() or delta.shape != h.shape)):
-        raise ValueError("h and delta must be contiguous and of one shape")
-    if weight.shape != (hidden,) or weight.dtype != h.dtype or (delta is not None and delta.dtype != h.dtype):
-        raise ValueError("weight must be (hidden,) and every operand of h's dtype")
-    if out is None:
-        out = torch.empty_like(h)
-    elif out.shape != h.shape or not out.is_contiguous() or out.dtype != h.dtype:
-        raise ValueError("out must be contiguous, of h's shape and dtype")
-    if delta is not None and h_out is None:
-        h_out = torch.empty_like(h)
-    elif h_out is not None and (h_out.shape != h.shape or not h_out.is_contiguous() or h_out.dtype != h.dtype):
-        raise ValueError("h_out must be contiguous, of h's shape and dtype")
-    n_rows = h.numel() // hidden if hidden else 0
-    check(
-        lib().ckv_add_rmsnorm(
-            _ptr(h_out), _ptr(h), _ptr(delta), _ptr(out), _ptr(weight.contiguous()), n_rows, hidden, float(eps),
-            dtype_code(h.dtype), _stream(h.device),
-        ),
-        "ckv_add_rmsnorm",
-    )
-    return (h if delta is None else h_out), out
+    return _native.torch_ops().add_rmsnorm(h, delta, weight, eps, h_out, out)
 
 
 def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """silu(gate) * up with the MLP's roundings (torch_engine.py:72 via the SiLU-gated Qwen2/Llama
     MLP). gate/up: (..., width) with evenly spaced contiguous rows (e.g. the halves of one
     stacked GEMM output); returns a contiguous (..., width) tensor."""
-    _dev(gate, up)
-    width = gate.shape[-1]
-    if up.shape != gate.shape or up.dtype != gate.dtype:
-        raise ValueError("gate and up must have one shape and dtype")
-    gs, us = _row_major(gate, width, "gate"), _row_major(up, width, "up")
-    if out is None:
-        out = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
-    elif out.shape != gate.shape or not out.is_contiguous() or out.dtype != gate.dtype:
-        raise ValueError("out must be contiguous, of gate's shape and dtype")
-    n_rows = gate.numel() // width if width else 0
-    check(
-        lib().ckv_silu_mul(
-            _ptr(out), width, _ptr(gate), gs, _ptr(up), us, n_rows, width, dtype_code(gate.dtype), _stream(gate.device),
-        ),
-        "ckv_silu_mul",
-    )
-    return out
+    return _native.torch_ops().silu_mul(gate, up, out)

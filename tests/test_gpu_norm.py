@@ -122,3 +122,30 @@ def test_fused_ops_reject_bad_layouts():
     g = torch.zeros(4, 64, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(ValueError):
         ops.silu_mul(g[:, 1:57], g[:, 1:57])  # rows not 16-byte aligned
+
+
+@pytest.mark.parametrize("view,ok", [
+    (lambda b: b[..., :32], True),             # halves of a stacked product
+    (lambda b: b[..., 32:], True),
+    (lambda b: b[1:2, 2:5, :32], True),
+    (lambda b: b[:, ::2, :32], True),          # every second row: still evenly spaced
+    (lambda b: b[:0, :, :32], True),           # no rows
+    (lambda b: b[0, 0, :32], True),            # one row, no row dimension
+    (lambda b: b[:, :5, :32], False),          # a gap between the outer rows
+    (lambda b: b[:1, :, :32].expand(4, 6, 32), False),   # repeated rows, outer and inner
+    (lambda b: b[:, :1, :32].expand(4, 6, 32), False),
+    (lambda b: b[:1, :1, :32].expand(4, 6, 32), False),
+    (lambda b: b[0, :1, :32].expand(6, 32), False),
+    (lambda b: b.transpose(1, 2)[:, :32], False),        # columns apart
+    (lambda b: b[..., 1:33], False),           # rows off their 16-byte boundary
+])
+def test_gated_product_row_layouts(view, ok):
+    """Row layouts that silu_mul takes (each equal to the contiguous copy's result) and refuses."""
+    b = torch.randn(4, 6, 64, generator=torch.Generator().manual_seed(1)).to("cuda", torch.bfloat16)
+    g = view(b)
+    if not ok:
+        with pytest.raises(ValueError):
+            ops.silu_mul(g, g)
+        return
+    out = ops.silu_mul(g, g)
+    assert out.is_contiguous() and torch.equal(out, ops.silu_mul(g.contiguous(), g.contiguous()))
