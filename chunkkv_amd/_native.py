@@ -97,6 +97,8 @@ SIGNATURES = {
     "ckv_attention_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32, _p, _p]),
     "ckv_add_rmsnorm": (_i32, [_p, _p, _p, _p, _p, _i64, _i32, _f32, _i32, _p]),
     "ckv_silu_mul": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i64, _i32, _i32, _p]),
+    "ckv_linear": (_i32, [_p, _p, _i64, _p, _p, _i32, _i32, _i32, _i32, _p, _i64, _p]),
+    "ckv_linear_workspace_bytes": (_i64, [_i32, _i32, _i32]),
     "ckv_scatter_rows": (
         _i32,
         [_p, _p, _i64, _p, _i64, _i64, _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _i32, _p, _p],

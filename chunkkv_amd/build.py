@@ -22,7 +22,8 @@ INCLUDE = ROOT / "include"
 LIB_DIR = PKG / "_lib"
 LIB_NAME = "libchunkkv_amd.so"
 SOURCES = ["abi.hip", "rerope_gather.hip", "assemble.hip", "deviation.hip", "select.hip", "select_gather.hip", "deviation_select.hip",
-           "scatter.hip", "layer1_repair.hip", "attention.hip", "rope.hip", "extract.hip", "norm.hip"]
+           "scatter.hip", "layer1_repair.hip", "attention.hip", "rope.hip", "extract.hip", "norm.hip",
+           "linear.hip"]
 HOST_SOURCES = ["token_hash.cpp"]
 TORCH_SOURCE, TORCH_OPS_NAME = "torch_ops.cpp", "_torch_ops.so"
 ARCH = "gfx950"

@@ -14,6 +14,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/types.h>
+#include <pybind11/pybind11.h>
 
 #include <algorithm>
 #include <cmath>
@@ -316,6 +317,43 @@ PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   CKV_PY_END
 }
 
+// linear(x, weight, bias): ckv_linear where it is the better choice and takes the operands, else torch's
+PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
+  CKV_PY_BEGIN
+  need_args(n_args, 3);
+  const Tensor &x = tensor(a[0]), &w = tensor(a[1]), bias = optional_tensor(a[2]);
+  auto plain = [&](const Tensor& t) {
+    return t.is_cuda() && t.device() == x.device() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
+           (uintptr_t)t.data_ptr() % 16 == 0 && !(at::GradMode::is_enabled() && t.requires_grad());
+  };
+  int64_t ws_bytes = -1;
+  if (x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && w.numel() > 0 && x.numel() > 0 && plain(x) && plain(w) &&
+      (!bias.defined() || (bias.dim() == 1 && bias.size(0) == w.size(0) && plain(bias)))) {
+    const int64_t rows = x.numel() / x.size(-1);
+    if (rows <= INT32_MAX && w.size(0) <= INT32_MAX && w.size(1) <= INT32_MAX)
+      ws_bytes = ckv_linear_workspace_bytes(int32(rows), int32(w.size(0)), int32(w.size(1)));
+  }
+  if (ws_bytes < 0) {
+    Tensor out;
+    {
+      pybind11::gil_scoped_release off;
+      out = at::linear(x, w, bias.defined() ? std::optional<Tensor>(bias) : std::nullopt);
+    }
+    return THPVariable_Wrap(out);
+  }
+  at::DimVector shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = w.size(0);
+  Tensor out = at::empty(shape, x.options()), ws;
+  if (ws_bytes > 0) ws = at::empty({ws_bytes / 4}, x.options().dtype(at::kFloat));
+  check(unlocked([&] {
+          return ckv_linear(ptr(out), ptr(x), x.size(-1), ptr(w), ptr(bias), int32(x.numel() / x.size(-1)),
+                            int32(w.size(0)), int32(w.size(1)), CKV_DTYPE_BF16, ptr(ws), ws_bytes, stream_of(x));
+        }),
+        "ckv_linear");
+  return THPVariable_Wrap(out);
+  CKV_PY_END
+}
+
 // layer1_repair_gather(k_slab, v_slab, src_tab, layer, begin, end, segments, n_segs, max_seg_tokens, k, v, flags,
 //                      local, spans, threshold, theta, workspace, err, out, diff_norm) with out None or the six
 // tensors of a Selection and diff_norm None or two: (diff, norm, the six tensors)
@@ -464,6 +502,7 @@ PyMethodDef kMethods[] = {
     {"rope_qkv", (PyCFunction)(void (*)(void))rope_qkv, METH_FASTCALL, nullptr},
     {"add_rmsnorm", (PyCFunction)(void (*)(void))add_rmsnorm, METH_FASTCALL, nullptr},
     {"silu_mul", (PyCFunction)(void (*)(void))silu_mul, METH_FASTCALL, nullptr},
+    {"linear", (PyCFunction)(void (*)(void))linear, METH_FASTCALL, nullptr},
     {"layer1_repair_gather", (PyCFunction)(void (*)(void))layer1_repair_gather, METH_FASTCALL, nullptr},
     {"extract_chunks", (PyCFunction)(void (*)(void))extract_chunks, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};

@@ -133,6 +133,16 @@ def _stack_params(mods: list, name: str) -> torch.Tensor | None:
     return stacked
 
 
+def _apply_linear(m, x: torch.Tensor) -> torch.Tensor:
+    """m(x); for an nn.Linear that nothing wraps, hooks or patches, its product by ops.linear."""
+    if (type(m) is torch.nn.Linear and not m._forward_hooks and not m._forward_pre_hooks
+            and "forward" not in m.__dict__ and not torch.nn.modules.module._has_any_global_hook()):
+        w = m._parameters.get("weight")
+        if w is not None:
+            return ops.linear(x, w, m._parameters.get("bias"))
+    return m(x)
+
+
 class HipEngine(DecoderPieces):
     def __init__(self, model, tokenizer, attention: str = "fused", overlap: bool = False,
                  layer1: str = "one_call"):
@@ -239,9 +249,9 @@ class HipEngine(DecoderPieces):
             return h + layer.mlp(layer.post_attention_layernorm(h)), None
         w, eps = self._norm_post[li]
         h, x = ops.add_rmsnorm(h, a, w, eps, h_out=h)
-        gu = F.linear(x, self._w_gu[li], self._b_gu[li])
+        gu = ops.linear(x, self._w_gu[li], self._b_gu[li])
         width = gu.shape[-1] // 2
-        return h, layer.mlp.down_proj(ops.silu_mul(gu[..., :width], gu[..., width:]))
+        return h, _apply_linear(layer.mlp.down_proj, ops.silu_mul(gu[..., :width], gu[..., width:]))
 
     def _final_logits(self, h, pending):
         """lm_head(norm(h + pending)) of the given rows (torch_engine.py:75)."""
@@ -270,7 +280,7 @@ class HipEngine(DecoderPieces):
         if self._native_attention and self.attention == "fused":
             # positions-only mask on the matrix-core kernel; output already token-major
             o = ops.attention_active(q, K, V, active, err=err)
-            return self._mlp(li, layer, h, attn.o_proj(o.view(h.shape[0], h.shape[1], -1)))
+            return self._mlp(li, layer, h, _apply_linear(attn.o_proj, o.view(h.shape[0], h.shape[1], -1)))
         group = self.n_heads // self.n_kv
         if self.attention == "sdpa":
             # torch's fused kernels only: K/V repeated per query group (their GQA form), the
@@ -376,7 +386,7 @@ class HipEngine(DecoderPieces):
 
     def _project(self, li: int, x: torch.Tensor):
         """q|k|v projection of layer li in one GEMM: views (1, n, H*D) of its token-major output."""
-        lin = F.linear(x, self._w_qkv[li], self._b_qkv[li])
+        lin = ops.linear(x, self._w_qkv[li], self._b_qkv[li])
         qd, kd = self.n_heads * self.head_dim, self.n_kv * self.head_dim
         return lin[..., :qd], lin[..., qd : qd + kd], lin[..., qd + kd :]
 

@@ -707,3 +707,9 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
     MLP). gate/up: (..., width) with evenly spaced contiguous rows (e.g. the halves of one
     stacked GEMM output); returns a contiguous (..., width) tensor."""
     return _native.torch_ops().silu_mul(gate, up, out)
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+    """torch.nn.functional.linear(x, weight, bias): on ckv_linear for the bf16 projections of short
+    requests (contiguous operands, no gradient asked for), on torch's library call for the rest."""
+    return _native.torch_ops().linear(x, weight, bias)

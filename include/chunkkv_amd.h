@@ -572,6 +572,26 @@ int32_t ckv_silu_mul(void* out, int64_t out_row_stride, const void* gate, int64_
                      void* stream);
 
 /*
+ * out = x W^T + bias, the function of nn.Linear: x (n_rows, n_in) with rows x_row_stride elements
+ * apart (a multiple of 8), weight (n_out, n_in) contiguous, bias (n_out) or NULL, out (n_rows, n_out)
+ * contiguous; bf16, 16-byte aligned, n_in a multiple of 64 and n_out of 8. Products and the bias add
+ * accumulate in fp32, one rounding at the end. Made for the projections of short requests;
+ * ckv_linear_workspace_bytes says for which.
+ *   workspace  optional device buffer of workspace_bytes >= ckv_linear_workspace_bytes(...)
+ *              (16-byte aligned): with it, products whose tiles leave the chip idle split n_in and
+ *              sum the fp32 partials in order; without it they run unsplit (the same up to the
+ *              order of fp32 sums).
+ * Replaces: the projections of torch_engine.py:61-72 (the modules' own GEMM calls).
+ */
+int32_t ckv_linear(void* out, const void* x, int64_t x_row_stride, const void* weight, const void* bias,
+                   int32_t n_rows, int32_t n_out, int32_t n_in, int32_t dtype, void* workspace,
+                   int64_t workspace_bytes, void* stream);
+
+/* Bytes of workspace that ckv_linear uses for this shape (0: it does not split it), or -1 where the
+ * libraries' GEMMs are the better choice or ckv_linear does not take the shape. Host-only. */
+int64_t ckv_linear_workspace_bytes(int32_t n_rows, int32_t n_out, int32_t n_in);
+
+/*
  * Token-prefix hashes (host memory, host code): digests[32*i .. 32*i + 32) = SHA-256 of the
  * message LE32(s) || LE32(tokens[0]) || ... || LE32(tokens[s - 1]) with s = starts[i], i.e.
  * the reference's keys.token_hash(tokens[:s]) as raw bytes (its hexdigest is their hex).
