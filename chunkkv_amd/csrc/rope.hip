@@ -14,7 +14,8 @@
 // from theta, passed by value in the kernel arguments) and each token's position, evaluated in
 // fp64 with the short reduction + series of cos_sin.hpp. A k/v-only launch (the cache repair)
 // runs one wavefront per token, each lane evaluating one frequency once and the lanes sharing
-// them through ds_bpermute; a launch with q shares each evaluation over 4 heads. A caller-kept
+// them through ds_bpermute, and so does a launch with q (head_dim 256: each evaluation shared over 4
+// heads). A caller-kept
 // per-position table (ckv_rope_table) is also accepted. All accesses are 16 bytes. The ~20 elementwise torch
 // launches of the reference's RoPE (fp32 temporaries, cat, cast) and the separate scatter of k/v
 // into the cache become one pass over the projection output.
@@ -291,7 +292,89 @@ __global__ __launch_bounds__(kRopeKvThreads) void rope_kv_kernel(
   }
 }
 
-// Without a table, with q (32+ rotated heads share each token's cos/sin): one thread per
+// Without a table, with q, head_dim <= 128: one wavefront per token, as rope_kv_kernel. Item i of a
+// token is the 16-byte column pair (col, col + D/2) of head row i / TPR: q heads, then k heads
+// (rotated), then v heads (copied); lane l takes items l, l + 64, ... and its first NB items' loads
+// all go out before the cos/sin are built, so that a token of up to NB x 64 items costs one round
+// trip (more items follow in batches of NB). Lane f evaluates frequency f once for all the token's
+// heads; the form before shared an evaluation over four heads only, eight to a thread, and divided
+// integers per item. Bound: one round trip at small launches, HBM at large ones. Measured (us, graph
+// replays, the form before first): 28 + 4 heads of 128, 251 tokens 5.2 -> 4.4, 2976 12.0 -> 10.8, 8256
+// 35.0 -> 31.4 (4.8 TB/s); 14 + 2 heads of 64, 251 tokens 5.0 -> 2.9, 8256 10.7 -> 8.7, in fp32 13.2
+// -> 12.5. Loads stay regular: non-temporal ones took 27.4 us for the largest but 9.8 and 14.9 for
+// the two others (the projection's output is usually still in a cache).
+template <int DTYPE, int D, int RM, int NB>
+__global__ __launch_bounds__(kRopeKvThreads) void rope_token_kernel(
+    int n, int Hq, int Hkv, int items, const int64_t* __restrict__ pos, const char* __restrict__ q_in,
+    const char* __restrict__ k_in, const char* __restrict__ v_in, int64_t qi_hs_b, int64_t qi_ts_b, int64_t ki_hs_b,
+    int64_t ki_ts_b, int64_t vi_hs_b, int64_t vi_ts_b, char* __restrict__ q_out, char* __restrict__ k_out,
+    char* __restrict__ v_out, int64_t qo_hs_b, int64_t qo_ts_b, int64_t ko_hs_b, int64_t ko_ts_b, int64_t vo_hs_b,
+    int64_t vo_ts_b, const int64_t* __restrict__ rows, int n_out, int32_t* __restrict__ err, const InvFreq inv) {
+  using E = Elem<DTYPE>;
+  constexpr int VEC = E::kVec;
+  constexpr int HALF = D / 2;
+  constexpr int TPR = HALF / VEC;  // column pairs per head row (a power of two)
+  constexpr int HALF_B = HALF * E::kBytes;
+  static_assert(HALF <= kWave && kWave % HALF == 0 && (TPR & (TPR - 1)) == 0, "head_dim out of range");
+  const int lane = threadIdx.x & (kWave - 1);
+  const int t = (int)blockIdx.x;
+  const int64_t p = pos[t];
+  const int64_t row = RM == kRowToken ? (int64_t)t : RM == kRowPos ? p : rows[t];
+  const int col = lane & (TPR - 1);
+  const int n_rk = Hq + Hkv;
+  auto src_of = [&](int it) {
+    const int h = it / TPR;
+    const char* b = h < Hq     ? q_in + h * qi_hs_b + t * qi_ts_b
+                    : h < n_rk ? k_in + (h - Hq) * ki_hs_b + t * ki_ts_b
+                               : v_in + (h - n_rk) * vi_hs_b + t * vi_ts_b;
+    return b + col * 16;
+  };
+  vec16 a[NB], b[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {  // a lane past the end loads the last item again
+    const char* s = src_of(min(lane + j * kWave, items - 1));
+    a[j] = ld16(s);
+    b[j] = ld16(s + HALF_B);
+  }
+  const bool ok = p >= INT32_MIN && p <= INT32_MAX && row >= 0 && row < n_out;
+  float ang[1] = {(float)(ok ? (int)p : 0) * inv.v[lane & (HALF - 1)]}, cv[1], sv[1];
+  angles_cos_sin<1>(ang, cv, sv);
+  if (!ok) {  // uniform
+    if (lane == 0) flag_error(err, CKV_DEVICE_ERR_RANGE);
+    return;
+  }
+  float c[VEC], sn[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    c[e] = __shfl(cv[0], col * VEC + e);
+    sn[e] = __shfl(sv[0], col * VEC + e);
+  }
+  for (int j0 = 0; j0 * kWave < items; j0 += NB) {
+    if (j0 > 0) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const char* s = src_of(min(lane + (j0 + j) * kWave, items - 1));
+        a[j] = ld16(s);
+        b[j] = ld16(s + HALF_B);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int it = lane + (j0 + j) * kWave, h = it / TPR;
+      if (it >= items) break;
+      char* d = (h < Hq     ? q_out + h * qo_hs_b + t * qo_ts_b
+                 : h < n_rk ? k_out + (h - Hq) * ko_hs_b + row * ko_ts_b
+                            : v_out + (h - n_rk) * vo_hs_b + row * vo_ts_b) +
+                col * 16;
+      vec16 y1 = a[j], y2 = b[j];
+      if (h < n_rk) rotate_pairs<DTYPE>(a[j], b[j], c, sn, y1, y2);
+      st16(d, y1);
+      st16(d + HALF_B, y2);
+    }
+  }
+}
+
+// Without a table, with q, head_dim 256: one thread per
 // (token, 16-byte column, group of kRopeFreeHG heads), grid-stride, evaluating its VEC
 // frequencies itself (kRopeFreeHG-fold sharing), v copied in 16-byte chunks. The thread's loads go
 // out in the order their values are needed (position, row, inverse frequencies, data) and it
@@ -503,13 +586,31 @@ static void launch_rope(int n, hipStream_t st, char* qo, int64_t qo_hs, int64_t 
                        ki_hs, ki_ts, vi, vi_hs, vi_ts, pos, inv, n, Hq, Hkv, err);
     return;
   }
-  using E = Elem<DTYPE>;
-  const int64_t per_tok = (int64_t)(Hq + Hkv + kRopeFreeHG - 1) / kRopeFreeHG * (D / 2 / E::kVec) +
-                          (vo != nullptr ? Hkv * (D * E::kBytes / 16) : 0);
-  const int64_t blocks = std::min<int64_t>((n * per_tok + kRopeThreads - 1) / kRopeThreads, 1 << 20);
-  hipLaunchKernelGGL((rope_free_kernel<DTYPE, D>), dim3((unsigned)blocks), dim3(kRopeThreads), 0, st, qo, qo_hs, qo_ts,
-                     ko, ko_hs, ko_ts, vo, vo_hs, vo_ts, rows, n_out, qi, qi_hs, qi_ts, ki, ki_hs, ki_ts, vi, vi_hs,
-                     vi_ts, pos, inv, n, Hq, Hkv, err);
+  if constexpr (D <= 2 * kWave) {
+    const int items = (Hq + Hkv + (vo != nullptr ? Hkv : 0)) * (D / 2 / Elem<DTYPE>::kVec);
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(kRopeKvThreads), 0, st, n, Hq, Hkv, items, pos, qi, ki, vi, qi_hs,
+                         qi_ts, ki_hs, ki_ts, vi_hs, vi_ts, qo, ko, vo, qo_hs, qo_ts, ko_hs, ko_ts, vo_hs, vo_ts, rows,
+                         n_out, err, inv);
+    };
+    auto batch = [&](auto nb) {
+      constexpr int NB = decltype(nb)::value;
+      if (rows == nullptr) go(rope_token_kernel<DTYPE, D, kRowToken, NB>);
+      else if (rows == pos) go(rope_token_kernel<DTYPE, D, kRowPos, NB>);
+      else go(rope_token_kernel<DTYPE, D, kRowIndexed, NB>);
+    };
+    if (items <= 2 * kWave) batch(std::integral_constant<int, 2>{});
+    else if (items <= 3 * kWave) batch(std::integral_constant<int, 3>{});
+    else batch(std::integral_constant<int, 5>{});
+  } else {
+    using E = Elem<DTYPE>;
+    const int64_t per_tok = (int64_t)(Hq + Hkv + kRopeFreeHG - 1) / kRopeFreeHG * (D / 2 / E::kVec) +
+                            (vo != nullptr ? Hkv * (D * E::kBytes / 16) : 0);
+    const int64_t blocks = std::min<int64_t>((n * per_tok + kRopeThreads - 1) / kRopeThreads, 1 << 20);
+    hipLaunchKernelGGL((rope_free_kernel<DTYPE, D>), dim3((unsigned)blocks), dim3(kRopeThreads), 0, st, qo, qo_hs, qo_ts,
+                       ko, ko_hs, ko_ts, vo, vo_hs, vo_ts, rows, n_out, qi, qi_hs, qi_ts, ki, ki_hs, ki_ts, vi, vi_hs,
+                       vi_ts, pos, inv, n, Hq, Hkv, err);
+  }
 }
 
 typedef void (*RopeLaunch)(int, hipStream_t, char*, int64_t, int64_t, char*, int64_t, int64_t, char*, int64_t,

@@ -220,3 +220,35 @@ def test_rope_kv_every_row_mode_and_shape(shape, row_mode, n):
     Vw[:, rows] = _heads(vn, Hkv, D)
     np.testing.assert_array_equal(O.to_numpy(K)[0], Kw)
     np.testing.assert_array_equal(O.to_numpy(V)[0], Vw)
+
+
+@pytest.mark.parametrize("bf16,D,Hq,Hkv,n", [
+    (True, 64, 1, 1, 1),     # 12 of a wavefront's 64 items
+    (True, 128, 12, 2, 3),   # 128 items: exactly two a lane
+    (True, 128, 13, 2, 65),  # 136
+    (False, 64, 20, 2, 7),   # 192: exactly three
+    (True, 128, 28, 4, 129), # 288: the last of five part full
+    (True, 128, 32, 4, 5),   # 320: exactly five
+    (False, 128, 33, 8, 9),  # 784: batches after the first
+])
+def test_rope_qkv_items_per_token(bf16, D, Hq, Hkv, n):
+    """Every batch size of the one-wavefront-per-token kernel at its edges, in its three row modes
+    (row = token, row = position, indexed rows), bit for bit against the oracle."""
+    rng = np.random.default_rng(D + Hq + n)
+    lin = _proj(rng, n, Hq, Hkv, D, bf16)
+    N = n + 40
+    lt = O.from_numpy(lin, DEV)
+    q_in, k_in, v_in = _split(lt, Hq, Hkv, D)
+    qn, kn, vn = _split(lin, Hq, Hkv, D)
+    pos = rng.choice(N, n, replace=False).astype(np.int64)
+    pt = torch.from_numpy(pos).to(DEV)
+    for rows in (None, pt, torch.flip(pt, (0,)).contiguous()):
+        at = np.arange(n) if rows is None else rows.cpu().numpy()
+        K = torch.full((1, Hkv, N, D), -3.0, dtype=lt.dtype, device=DEV)
+        V = torch.full_like(K, -3.0)
+        q_out, _ = ops.rope_qkv(q_in, k_in, v_in, pt, Hq, Hkv, D, THETA, k_out=K, v_out=V, rows=rows)
+        np.testing.assert_array_equal(O.to_numpy(q_out)[0].transpose(1, 0, 2), O.rope(_heads(qn, Hq, D), pos, THETA))
+        np.testing.assert_array_equal(O.to_numpy(K)[0][:, at], O.rope(_heads(kn, Hkv, D), pos, THETA))
+        np.testing.assert_array_equal(O.to_numpy(V)[0][:, at], _heads(vn, Hkv, D))
+        rest = np.setdiff1d(np.arange(N), at)
+        assert bool((K[0][:, rest] == -3).all()) and bool((V[0][:, rest] == -3).all())
