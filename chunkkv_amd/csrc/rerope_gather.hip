@@ -18,17 +18,17 @@
 
 namespace ckv {
 
-// Launch shapes (threads, tokens per tile, row slots in flight per thread, grid order), measured
-// on MI355X at the Qwen2.5-7B KV shape (4 heads x 128, bf16).
-//  - Tile-fastest grid (x = tile, y = segment): the workgroups in flight together stream
-//    neighbouring tiles of one segment. Dense gathers (every row of a segment): 256 threads x 8
-//    tokens x 2 slots. Gathers with a skip map (a selection leaves rows out at scattered
-//    positions): 512 x 16 x 1; the 8k request's dropped rows of 26 layers (24 segments) take
-//    95 us, against 112 us with the segment-fastest grid, and 108 / 114 us with 256 threads x
-//    16 tokens x 2 slots / 32 tokens x 4 slots.
-//  - Segment-fastest grid (x = segment, y = tile), 256 x 16 x 4, for launches of 64 segments or
-//    more: the replay's 4 concurrent 32k requests (128 segments each) reach 75.0 % of HBM peak
-//    with it, 68.2 % with the tile-fastest shapes above.
+// Launch shapes (threads, tokens per tile, row slots in flight per thread), measured on MI355X at
+// the Qwen2.5-7B KV shape (4 heads x 128, bf16). The grid is x = tile, y = segment: the workgroups
+// in flight together stream neighbouring tiles of one segment.
+//  - Dense gathers (every row of a segment): 256 threads x 8 tokens x 2 slots.
+//  - Gathers with a skip map (a selection leaves rows out at scattered positions): 512 x 16 x 1; the
+//    8k request's dropped rows of 26 layers (24 segments) take 95 us, against 112 us with x =
+//    segment, and 108 / 114 us with 256 threads x 16 tokens x 2 slots / 32 tokens x 4 slots.
+//  - Launches of 64 segments or more: 256 x 16 x 4. One 32,832-token request's repair (128 segments)
+//    takes 768 us, against 801 with x = segment, 772 with the skip shape (non-temporal stores), 780
+//    with 2 slots, 784-805 with 512 threads; four of them on four streams 2.88 ms a round against
+//    2.91-2.93 with x = segment and 3.00 with the skip shape.
 // Stores (a StorePolicy per shape; rows are loaded non-temporally by every shape): the skip and
 // dense shapes store the key rows with device scope (sc1: written through the L2, nothing of
 // them left for the end-of-launch writeback) and the value rows with device scope and
@@ -38,24 +38,25 @@ namespace ckv {
 // us; earlier: 98.5 us with both non-temporal, 112.0 us both regular); config 2's dense gather
 // 77.3-77.9 against 77.8-78.3 us with both non-temporal; config 5's rounds 2.908-2.919 ms with
 // both non-temporal against 3.015-3.024 ms with either device-scope form.
-struct GatherDense {
+struct GatherDense {  // below kGatherWideSegs segments, as the next
+  static constexpr bool kManySegs = false;
   static constexpr int kThreads = 256, kTile = 8, kUnroll = 2;
-  static constexpr bool kSegFastest = false;
   static constexpr int kStK = kStAgent, kStV = kStAgentStream;
 };
 struct GatherSkip {
+  static constexpr bool kManySegs = false;
   static constexpr int kThreads = 512, kTile = 16, kUnroll = 1;
-  static constexpr bool kSegFastest = false;
   static constexpr int kStK = kStAgent, kStV = kStAgentStream;
 };
 struct GatherWide {
+  static constexpr bool kManySegs = true;  // possibly more than grid y holds
   static constexpr int kThreads = 256, kTile = 16, kUnroll = 4;
-  static constexpr bool kSegFastest = true;
   static constexpr int kStK = kStStream, kStV = kStStream;
 };
 constexpr int kGatherWideSegs = 64;  // segment count from which GatherWide is used
+constexpr int kGridYZ = 65535;       // most blocks in y and z
 
-// Grid: (tile, segment) in the order of S (x fastest), z = layer. With ROWS, the first scat_z
+// Grid: x = tile, y = segment (seg_x: the other way round, for more segments than y holds), z = layer. With ROWS, the first scat_z
 // z-slices scatter rows (another layer's kept rows, rs) instead, items grid-stride over them:
 // dispatched first, they run beside the gather's first tiles.
 template <int DTYPE, int D, class S, bool ROWS>
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(S::kThreads) void rerope_gather_kernel(
     const ckv_segment* __restrict__ segs, ckv_segment one_seg, uint64_t one_src_k,
     uint64_t one_src_v, int64_t one_src_head_stride_b, int n_layers, int layer_begin, int n_heads,
     int n_tokens, const int32_t* __restrict__ skip, const InvFreq inv, int32_t* __restrict__ err,
-    const RowScatter rs, int scat_z) {
+    const RowScatter rs, int scat_z, int seg_x) {
   int zl = (int)blockIdx.z;
   if constexpr (ROWS) {
     if (zl < scat_z) {  // uniform: a scatter block
@@ -81,10 +82,11 @@ __global__ __launch_bounds__(S::kThreads) void rerope_gather_kernel(
     }
     zl -= scat_z;
   }
+  const bool sx = S::kManySegs && seg_x;
   gather_tile<DTYPE, D, S::kThreads, S::kTile, S::kUnroll, true, S::kStK, S::kStV>(
       dst_k, dst_v, dst_layer_stride_b, dst_head_stride_b, src_tab, n_chunks, segs,
-      (int)(S::kSegFastest ? blockIdx.x : blockIdx.y), one_seg, one_src_k, one_src_v, one_src_head_stride_b, n_layers,
-      layer_begin + zl, (int)(S::kSegFastest ? blockIdx.y : blockIdx.x), n_heads, n_tokens, skip, inv, err);
+      (int)(sx ? blockIdx.x : blockIdx.y), one_seg, one_src_k, one_src_v, one_src_head_stride_b, n_layers,
+      layer_begin + zl, (int)(sx ? blockIdx.y : blockIdx.x), n_heads, n_tokens, skip, inv, err);
 }
 
 // Writes the D/2 inverse frequencies the kernels above take in their arguments.
@@ -110,15 +112,16 @@ static void launch_gather(char* dk, char* dv, int64_t ls_b, int64_t hs_b, const 
       scat_z = (int)std::min<int64_t>(std::max<int64_t>(1, (items + 2 * per_z - 1) / (2 * per_z)), 1024);
     }
     const unsigned zs = (unsigned)(layer_count + scat_z);
-    const dim3 grid = S::kSegFastest ? dim3((unsigned)n_segs, tiles, zs) : dim3(tiles, (unsigned)n_segs, zs);
+    const int seg_x = n_segs > kGridYZ;
+    const dim3 grid = seg_x ? dim3((unsigned)n_segs, tiles, zs) : dim3(tiles, (unsigned)n_segs, zs);
     if (rs != nullptr)
       hipLaunchKernelGGL((rerope_gather_kernel<DTYPE, D, S, true>), grid, dim3(S::kThreads), 0, st, dk, dv, ls_b, hs_b,
                          tab, n_chunks, segs, one, one_k, one_v, one_hs_b, n_layers, layer_begin, n_heads, n_tokens,
-                         skip, host_inv_freq(D, theta), err, *rs, scat_z);
+                         skip, host_inv_freq(D, theta), err, *rs, scat_z, seg_x);
     else
       hipLaunchKernelGGL((rerope_gather_kernel<DTYPE, D, S, false>), grid, dim3(S::kThreads), 0, st, dk, dv, ls_b,
                          hs_b, tab, n_chunks, segs, one, one_k, one_v, one_hs_b, n_layers, layer_begin, n_heads,
-                         n_tokens, skip, host_inv_freq(D, theta), err, RowScatter{}, 0);
+                         n_tokens, skip, host_inv_freq(D, theta), err, RowScatter{}, 0, seg_x);
   };
   if (n_segs >= kGatherWideSegs) go(GatherWide{});
   else if (skip != nullptr) go(GatherSkip{});
@@ -178,8 +181,8 @@ int32_t gather_layers_launch(void* dst_k, void* dst_v, int64_t dst_layer_stride,
     n_segs = 1;
     layer_end = layer_begin;
   }
-  // grid y (tiles of the segment-fastest shape, segments below kGatherWideSegs) and z (layers)
-  if ((max_seg_tokens + 15) / 16 > 65535 || layer_end - layer_begin > 64000) return CKV_ERR_TOO_LARGE;
+  // grid y (segments, or tiles where there are more segments than that) and z (layers)
+  if ((max_seg_tokens + 15) / 16 > kGridYZ || layer_end - layer_begin > 64000) return CKV_ERR_TOO_LARGE;
   const int64_t eb = elem_bytes(dtype);
   fn((char*)dst_k, (char*)dst_v, dst_layer_stride * eb, dst_head_stride * eb, src_tab, n_chunks, segs, ckv_segment{},
      0, 0, 0, n_segs, max_seg_tokens, n_layers, layer_begin, layer_end - layer_begin, n_heads, n_tokens, skip, theta, err,

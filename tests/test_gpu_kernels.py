@@ -215,7 +215,7 @@ def test_rerope_gather_skip_map_uneven_selection(lens, pattern):
 
 @pytest.mark.parametrize("bf16,D", [(True, 128), (False, 64)])
 def test_rerope_gather_many_segments(bf16, D):
-    """Launches of 64 or more segments take the segment-fastest launch shape: 80 ragged segments
+    """Launches of 64 or more segments take a launch shape of their own: 80 ragged segments
     (1-40 tokens), every layer without a skip map and layers 1-2 with one, against the oracle."""
     rng = np.random.default_rng(640 + D)
     n_layers, H = 3, 2
@@ -320,6 +320,29 @@ def test_rerope_gather_config2_full_size():
     assert O.rerope_gather(Ko, Vo, okl, ovl, segs, THETA) == 0
     np.testing.assert_array_equal(host(V).reshape(Vo.shape), Vo)
     assert_keys_close(host(K).reshape(Ko.shape), Ko, True)
+
+
+@pytest.mark.parametrize("n_segs", [63, 64, 65535, 65536])
+def test_rerope_gather_segment_count_limits(n_segs):
+    """One-row segments at the counts where the launch shape and the grid's order change (64
+    segments, the 65,535 blocks of grid y): every row lands, bit for bit."""
+    H, D, L = 1, 64, 32
+    rng = np.random.default_rng(n_segs)
+    k, v = (O.f32_to_bf16_bits(rng.standard_normal((H, L, D)).astype(np.float32)) for _ in range(2))
+    kt, vt = O.from_numpy(k, DEV), O.from_numpy(v, DEV)
+    i = np.arange(n_segs)
+    segs = np.stack([i, np.ones_like(i), np.zeros_like(i), i % L, np.full_like(i, L), i % 7 * 100], 1).astype(np.int32)
+    tab = torch.tensor([kt.data_ptr(), vt.data_ptr()], dtype=torch.int64, device=DEV)
+    K = torch.zeros((1, 1, H, n_segs, D), dtype=torch.bfloat16, device=DEV)
+    V = torch.zeros_like(K)
+    err = torch.zeros(1, dtype=torch.int32, device=DEV)
+    ops.rerope_gather(K, V, tab, torch.from_numpy(segs.reshape(-1)).to(DEV), n_segs, 1, THETA, err)
+    assert int(err.item()) == 0
+    Ko, Vo = np.zeros((1, H, n_segs, D), dtype=np.uint16), np.zeros((1, H, n_segs, D), dtype=np.uint16)
+    assert O.rerope_gather(Ko, Vo, [[k]], [[v]], segs, THETA) == 0
+    np.testing.assert_array_equal(O.to_numpy(K)[:, 0], Ko)
+    np.testing.assert_array_equal(O.to_numpy(V)[:, 0], Vo)
+
 
 
 def test_rerope_gather_flags_bad_segment_without_writing():
