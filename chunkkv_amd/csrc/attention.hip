@@ -22,6 +22,16 @@
 // few 128-query workgroups to fill the chip (decode, short prompts, small blends) run
 // attention_wave.hpp's kernel instead. Built with the MFMA VGPR form (no accumulator-register
 // copies around the online-softmax rescale).
+// Bound: issue and power together. The matrix cores run half of the cycles and the vector
+// instructions most of the rest, so every vector instruction that is not softmax costs time: tile
+// addresses are a kept offset on a uniform base (62 -> 8 instructions a tile), wavefront extremes
+// are scalar (branches, not selects), the four lanes of a query agree on its max only where a lane
+// asks to raise it. Measured (us, 28 heads of 128): 2976 rows over 8256 216 -> 196 (1010 TFLOP/s),
+// 8256 causal rows 480 -> 449 (1089), 2000 51.2 -> 47.4; 14 heads of 64, 8256 causal rows 162 -> 144.
+// A square bf16 product of 8192 reaches 1300-1400 on this card; inputs of zeros (no toggling) 10 %
+// more than these. Not faster: tiles one ahead so that the matrix cores work beside the exponentials
+// (209-214 / 478 before this form, with spills), V operands read ahead of their products (the same),
+// eight wavefronts on one tile (233 / 476), 48 or 64 queries a wavefront (275 / 453, 322 / 649).
 #include <algorithm>
 
 #include "ckv_common.hpp"
@@ -49,11 +59,17 @@ __device__ __forceinline__ float group_max(float v) {
   auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-__device__ __forceinline__ float group_sum(float v) {  // fp32 addition commutes: every lane agrees
-  auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-  auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+// f over the 16 lanes of a row, in every lane (row rotations: VALU, no LDS round trip).
+template <typename T, typename F>
+__device__ __forceinline__ T row16_reduce(T v, F f) {
+  static_assert(sizeof(T) == 4, "one VGPR");
+  auto from = [](T x, auto ctrl) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
+  };
+  v = f(v, from(v, std::integral_constant<int, 0x128>{}));
+  v = f(v, from(v, std::integral_constant<int, 0x124>{}));
+  v = f(v, from(v, std::integral_constant<int, 0x122>{}));
+  return f(v, from(v, std::integral_constant<int, 0x121>{}));
 }
 
 typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -97,12 +113,6 @@ __device__ __forceinline__ bf16x8 v_operand(const char* vb, int dt, int g, int l
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-#ifndef CKV_ATTN_PRIO
-#define CKV_ATTN_PRIO 0  // 1: raise the wavefront's issue priority around its matrix-core sections
-#endif
-#ifndef CKV_ATTN_MFMA_SUM
-#define CKV_ATTN_MFMA_SUM 1  // softmax row sums on the matrix cores (a ones operand) instead of VALU adds
-#endif
 constexpr int kXcds = 8;  // MI355X: workgroups go round-robin to 8 XCDs, each with its own L2
 
 // Which work item (query block qb, head h, cache split z) a workgroup takes. The hardware hands
@@ -179,7 +189,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   __shared__ __attribute__((aligned(1024))) char v_lds1[kAttnBN * ROWB];
   __shared__ int blk_max_s[kAttnWaves];
 
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
   const int g = lane / 16, lm = lane % 16;
   int qb, hq, z;
   if (!attn_work_item(nqb, map_group, xpk_log, items, inv_group, inv_nqb, qb, hq, z)) return;
@@ -206,16 +216,14 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
     my_pos[qg] = p;
     wmax = max(wmax, p);
   }
-#pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) {
-    wmax = max(wmax, __shfl_xor(wmax, s, 64));
-    wmin = min(wmin, __shfl_xor(wmin, s, 64));
-  }
+  wmax = __builtin_amdgcn_readfirstlane(row16_reduce(wmax, [](int a, int b) { return max(a, b); }));
+  wmin = __builtin_amdgcn_readfirstlane(row16_reduce(wmin, [](int a, int b) { return min(a, b); }));
   if (lane == 0) blk_max_s[wave] = wmax;
   __syncthreads();
   int bmax = blk_max_s[0];
 #pragma unroll
   for (int w = 1; w < kAttnWaves; ++w) bmax = max(bmax, blk_max_s[w]);
+  bmax = __builtin_amdgcn_readfirstlane(bmax);
   const int n_tiles = bmax < 0 ? 0 : bmax / kAttnBN + 1;
 
   // Q fragments (B operand of S^T): query q0 + 16 qg + lm, head-dim 32 s + 8 g .. + 8.
@@ -232,9 +240,8 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   }
 
   f32x4 o[kAttnQG][DT];
-  float m_run[kAttnQG], l_run[kAttnQG];
-  // With CKV_ATTN_MFMA_SUM the row sums come from one more MFMA per key block with an all-ones A
-  // operand: every row of its output is sum_k P^T[k][query], the sum of the bf16 weights that
+  float m_run[kAttnQG], m_sub[kAttnQG];
+  // The row sums come from one more MFMA per key block with an all-ones A operand: every row of its output is sum_k P^T[k][query], the sum of the bf16 weights that
   // multiply V (lane (g, lm) gets query lm's sum in each of its four values).
   f32x4 l_acc[kAttnQG];
   const bf16x8 ones = {(__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f,
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
 #pragma unroll
   for (int qg = 0; qg < kAttnQG; ++qg) {
     m_run[qg] = -INFINITY;
-    l_run[qg] = 0.f;
+    m_sub[qg] = 0.f;
     l_acc[qg] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[qg][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -258,26 +265,39 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   // N - 1 instead (every query's position is below them, so they are masked).
   constexpr int KI = (kAttnBN * CPR) / NT;  // load instructions per wavefront, tile and tensor
   static_assert(KI >= 1 && (kAttnBN * CPR) % NT == 0, "a tile must fill whole load instructions");
-  int grow_k[KI], gcol_k[KI], gcol_v[KI];
+  // A lane's offsets in a tile are kept (K slots hold rows in kslot_row's order) and added to the
+  // tile's uniform address: two 64-bit addresses built per load were a quarter of a tile's vector
+  // instructions. Only a tile that reaches past the cache clamps its rows.
+  int off_k[KI], off_v[KI];
 #pragma unroll
   for (int i = 0; i < KI; ++i) {
     const int P = (wave * KI + i) * 64 + lane;
     const int slot = P / CPR, pc = P % CPR;
-    grow_k[i] = kslot_row(slot);
-    gcol_k[i] = (pc ^ swz_k<CPR>(slot)) * 16;
-    gcol_v[i] = (pc ^ swz_v<CPR>(slot)) * 16;
+    off_k[i] = kslot_row(slot) * ROWB + (pc ^ swz_k<CPR>(slot)) * 16;
+    off_v[i] = slot * ROWB + (pc ^ swz_v<CPR>(slot)) * 16;
   }
   typedef __attribute__((address_space(1))) void gvoid;
   typedef __attribute__((address_space(3))) void lvoid;
   auto issue = [&](int n0, char* kb, char* vb) {
+    const char* kt = kh + (int64_t)n0 * ROWB;
+    const char* vt = vh + (int64_t)n0 * ROWB;
+    const int last = N - 1 - n0;  // >= 0: only tiles that some query sees are issued
+    auto load = [&](const char* t, int off, char* to) {
+      __builtin_amdgcn_global_load_lds((gvoid*)(t + (uint32_t)off), (lvoid*)to, 16, 0, 0);
+    };
+    if (last >= kAttnBN - 1) {  // uniform: a whole tile
 #pragma unroll
-    for (int i = 0; i < KI; ++i) {
-      const int slot = ((wave * KI + i) * 64 + lane) / CPR;
-      const int rk = min(n0 + grow_k[i], N - 1), rv = min(n0 + slot, N - 1);
-      __builtin_amdgcn_global_load_lds((gvoid*)(kh + (int64_t)rk * ROWB + gcol_k[i]),
-                                       (lvoid*)(kb + (wave * KI + i) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((gvoid*)(vh + (int64_t)rv * ROWB + gcol_v[i]),
-                                       (lvoid*)(vb + (wave * KI + i) * 1024), 16, 0, 0);
+      for (int i = 0; i < KI; ++i) {
+        load(kt, off_k[i], kb + (wave * KI + i) * 1024);
+        load(vt, off_v[i], vb + (wave * KI + i) * 1024);
+      }
+    } else {
+      auto clamp = [&](int off) { return min(off / ROWB, last) * ROWB + off % ROWB; };
+#pragma unroll
+      for (int i = 0; i < KI; ++i) {
+        load(kt, clamp(off_k[i]), kb + (wave * KI + i) * 1024);
+        load(vt, clamp(off_v[i]), vb + (wave * KI + i) * 1024);
+      }
     }
   };
   // S^T operand of (kb, t, ds) for lane (g, lm): slot 32 kb + 16 t + lm, logical chunk 4 ds + g.
@@ -300,13 +320,12 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
     // S^T for the tile: lane (g, lm) gets query lm, rows n0 + 32 kb + 8 g + 4 t + e.
     constexpr int KB = kAttnBN / 32;
     f32x4 s[kAttnQG][KB][2];
-    if (CKV_ATTN_PRIO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
+      for (int ds = 0; ds < DS; ++ds) {  // the halves inside: dependent products four apart
 #pragma unroll
-        for (int ds = 0; ds < DS; ++ds) {
+        for (int t = 0; t < 2; ++t) {
           const bf16x8 a = *(const bf16x8*)(k_lds + (kb * 32 + 16 * t) * ROWB + k_rd[ds]);
 #pragma unroll
           for (int qg = 0; qg < kAttnQG; ++qg)
@@ -314,7 +333,6 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
                                                                                        : s[qg][kb][t], 0, 0, 0);
         }
       }
-    if (CKV_ATTN_PRIO) __builtin_amdgcn_s_setprio(0);
 
     // Online softmax over the tile. The running max is only raised when a query's tile max
     // exceeds it by more than 2^8 (log2 domain): weights stay <= 256, the output rescale is
@@ -345,34 +363,29 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int j = 0; j < 8; ++j) bm = fmaxf(bm, x[kb][j]);
-      bm = group_max(bm) * scale_log2;  // the scale is > 0: max commutes
-      const bool raise = bm > m_run[qg] + 8.f;  // also true on the first visible tile (m_run = -inf)
-      if (__builtin_amdgcn_ballot_w64(raise)) {  // uniform branch
+      // A lane asks for its own scores; the four lanes of a query agree on its max inside the branch.
+      if (__builtin_amdgcn_ballot_w64(bm * scale_log2 > m_run[qg] + 8.f)) {  // uniform branch
+        bm = group_max(bm) * scale_log2;           // the scale is > 0: max commutes
+        const bool raise = bm > m_run[qg] + 8.f;  // also true on the first visible tile (m_run = -inf)
         const float m_new = raise ? bm : m_run[qg];
         const float alpha = m_run[qg] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_run[qg] - m_new);
-        l_run[qg] *= alpha;
         l_acc[qg] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[qg][dt] *= alpha;
         m_run[qg] = m_new;
+        // with no visible row yet (absent queries) every score is -inf and subtracting 0 keeps p = 0
+        m_sub[qg] = m_new == -INFINITY ? 0.f : m_new;
       }
-      // p = 2^(score * scale - max) in one fma; with no visible row yet (absent queries) every
-      // score is -inf and subtracting 0 keeps p = 0.
-      const float msub = m_run[qg] == -INFINITY ? 0.f : m_run[qg];
-      float psum = 0.f;
+      // p = 2^(score * scale - max) in one fma
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(x[kb][e], scale_log2, -msub));
-          if (!CKV_ATTN_MFMA_SUM) psum += p;
-          pb[qg][kb][e] = (__bf16)p;
+          pb[qg][kb][e] = (__bf16)__builtin_amdgcn_exp2f(__builtin_fmaf(x[kb][e], scale_log2, -m_sub[qg]));
         }
-      if (!CKV_ATTN_MFMA_SUM) l_run[qg] += psum;
     }
 
     // O^T += V^T P^T: A = V^T rows dt*16 + lm, columns 32 kb + 8 g .. + 8.
-    if (CKV_ATTN_PRIO) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
@@ -381,13 +394,12 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
 #pragma unroll
         for (int qg = 0; qg < kAttnQG; ++qg)
           o[qg][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb[qg][kb], o[qg][dt], 0, 0, 0);
-        if (CKV_ATTN_MFMA_SUM && dt == DT - 1) {
+        if (dt == DT - 1) {
 #pragma unroll
           for (int qg = 0; qg < kAttnQG; ++qg)
             l_acc[qg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pb[qg][kb], l_acc[qg], 0, 0, 0);
         }
       }
-    if (CKV_ATTN_PRIO) __builtin_amdgcn_s_setprio(0);
   };
   for (int tile = 0; tile < n_tiles; tile += 2) {
     body(tile, k_lds0, v_lds0, k_lds1, v_lds1);
@@ -397,7 +409,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   // Normalise and write: lane (g, lm) holds O[query][dt*16 + 4g + e], 4 bf16 = 8 bytes per tile.
 #pragma unroll
   for (int qg = 0; qg < kAttnQG; ++qg) {
-    const float l = CKV_ATTN_MFMA_SUM ? l_acc[qg][0] : group_sum(l_run[qg]);
+    const float l = l_acc[qg][0];
     const int m = q0 + qg * 16 + lm;
     if (m >= n) continue;
     const float inv = 1.f / l;
@@ -435,12 +447,13 @@ struct AttnPlan {
   X(64, 1, 4, false) X(64, 1, 8, false) X(64, 2, 4, false) X(64, 2, 8, false)
 
 // Where the 128-query workgroups are too few: below about one for each of the 256 CUs at head_dim
-// 128 (us, 28 heads: 1103 causal rows, 252 workgroups, 27.7 against 29.5; 2000 rows, 448, 63.7
-// against 51.1), below two at head_dim 64, where they also hold less work each (14 heads: 4000
-// rows, 448 workgroups, 57.3 against 69.0; 6000, 658, 119 against 105).
+// 128 (us, 28 heads, this first: 768 causal rows, 168 workgroups, 19.7 against 20.6; 1000 of 8256
+// rows, 224, 157 against 164; 1103 causal rows, 252, 27.8 against 27.1; 1500, 336, 41.1 against
+// 36.5), below two at head_dim 64, where they also hold less work each (14 heads: 3000 causal rows,
+// 336 workgroups, 37.6 against 46.5; 4000, 448, 58.9 against 61.8; 4500, 504, 72.4 against 69.8).
 static bool wave_launch(int n, int Hq, int head_dim) {
   const int64_t blocks = (int64_t)((n + kAttnBM - 1) / kAttnBM) * Hq;
-  return blocks < (head_dim == 128 ? 256 : 512);
+  return blocks < (head_dim == 128 ? 256 : 450);
 }
 
 constexpr int kWaveFill = 256;  // workgroups that a split launch aims at: one for each CU

@@ -22,19 +22,6 @@
 
 namespace ckv {
 
-// f over the 16 lanes of a row, in every lane (row rotations: VALU, no LDS round trip).
-template <typename T, typename F>
-__device__ __forceinline__ T row16_reduce(T v, F f) {
-  static_assert(sizeof(T) == 4, "one VGPR");
-  auto from = [](T x, auto ctrl) {
-    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, false));
-  };
-  v = f(v, from(v, std::integral_constant<int, 0x128>{}));
-  v = f(v, from(v, std::integral_constant<int, 0x124>{}));
-  v = f(v, from(v, std::integral_constant<int, 0x122>{}));
-  return f(v, from(v, std::integral_constant<int, 0x121>{}));
-}
-
 template <int D, int QG, int W, bool GROUPED>
 __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
     int nqb, int map_group, int xpk_log, int items, uint32_t inv_group, uint32_t inv_nqb,

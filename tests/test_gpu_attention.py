@@ -146,7 +146,7 @@ def test_attention_small_launch_forms(Hq, Hkv, D, N, n):
     whole = ops.attention_active(*args, split=False)
     sub = np.unique(np.linspace(0, n - 1, min(n, 200)).astype(int))
     want = O.attention_active(q[:, sub], K[:, :seen], V[:, :seen], pos[sub])
-    small = -(-n // 128) * Hq < (256 if D == 128 else 512)
+    small = -(-n // 128) * Hq < (256 if D == 128 else 450)
     for out in (got, whole) if small else ():
         np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
     if not small:  # the large kernel multiplies zero weights into the rest of its last tile
