@@ -90,6 +90,7 @@ SIGNATURES = {
         _i32,
         [_p, _p, _i64, _i64, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _p, _p],
     ),
+    "ckv_extract_chunks_host": (_i32, [_p, _p, _i64, _i64, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32, _p]),
     "ckv_attention_active": (
         _i32,
         [_p, _p, _i64, _i64, _p, _p, _i64, _p, _i32, _i32, _i32, _i32, _i32, _i32, _f64, _p, _i64, _p, _p],

@@ -468,7 +468,24 @@ PyObject* extract_chunks(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     live += end > start;
     most = std::max(most, end - start);
   }
-  if (live > 0) {
+  const int code = live > 0 ? dtype_code(ks) : 0;
+  // Up to 64 segments go by value with the launch; a longer list goes through device memory.
+  if (live > 0 && live <= 64) {
+    uint64_t dst[64];
+    int32_t rows[128];
+    int32_t n = 0;
+    for (size_t i = 0; i < spans.size(); ++i) {
+      if (spans[i].second == spans[i].first) continue;
+      dst[n] = (uint64_t)(uintptr_t)bufs[i].data_ptr();
+      rows[2 * n] = (int32_t)spans[i].first;
+      rows[2 * n++ + 1] = (int32_t)(spans[i].second - spans[i].first);
+    }
+    check(unlocked([&] {
+            return ckv_extract_chunks_host(ptr(ks), ptr(vs), H * N * D, N * D, dst, rows, n, int32(L), int32(H), int32(N),
+                                           int32(D), code, stream_of(ks));
+          }),
+          "ckv_extract_chunks_host");
+  } else if (live > 0) {
     // descriptors: an address per span, then (start, length) pairs; pinned, one async copy (torch's
     // pinned allocator keeps the host block until the copy has run)
     Tensor host = at::empty({live * 2}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));
@@ -482,7 +499,6 @@ PyObject* extract_chunks(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
     }
     const Tensor d = host.to(ks.device(), /*non_blocking=*/true);
     const uint64_t* dst = (const uint64_t*)ptr(d);
-    const int code = dtype_code(ks);
     check(unlocked([&] {
             return ckv_extract_chunks(ptr(ks), ptr(vs), H * N * D, N * D, dst, (const int32_t*)(dst + live),
                                       int32(live), int32(most), int32(L), int32(H), int32(N), int32(D), code,

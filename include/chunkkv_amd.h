@@ -501,6 +501,16 @@ int32_t ckv_extract_chunks(const void* k_slab, const void* v_slab, int64_t layer
                            void* stream);
 
 /*
+ * ckv_extract_chunks with dst and spans in host memory, read before the call returns: they reach
+ * the kernel as its arguments, with no copy to the device. At most 64 spans (CKV_ERR_TOO_LARGE
+ * beyond); a span outside [0, n_tokens) is CKV_ERR_OUT_OF_RANGE and nothing is launched.
+ */
+int32_t ckv_extract_chunks_host(const void* k_slab, const void* v_slab, int64_t layer_stride,
+                                int64_t head_stride, const uint64_t* dst, const int32_t* spans,
+                                int32_t n_spans, int32_t n_layers, int32_t n_heads, int32_t n_tokens,
+                                int32_t head_dim, int32_t dtype, void* stream);
+
+/*
  * Attention of the active rows over the whole cache with the causal mask given by positions:
  *   out[i, h, :] = softmax_j( scale * q[h, i, :] . K[h / G, j, :] ) V[h / G, j, :],
  *   j ranging over [0, positions[i]], G = n_q_heads / n_kv_heads.

@@ -73,3 +73,32 @@ def test_prefill_result_chunk_uses_one_launch_and_matches_copies():
     # the extracted chunk is reusable at a new offset
     out = eng.prefill(toks[40:96] + toks[:8], [Placement(one, 0)], BlendConfig(recompute_ratio=0.3))
     assert out.stats["cached_tokens"] == 56
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 200])
+def test_extract_segment_count_limits(n):
+    """Up to 64 non-empty segments go with the launch's arguments, longer lists through device
+    memory: both are bit copies, empty spans in between, and lengths around the 8-token tile."""
+    L, H, N, D = 2, 3, 230, 64
+    g = torch.Generator(device=DEV).manual_seed(n)
+    K, V = (torch.randn((L, 1, H, N, D), generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    spans = []
+    for i in range(n):
+        spans += [(i, i + 1 + i % 17), (i, i)]
+    for (s, e), b in zip(spans, ops.extract_chunks(K, V, spans), strict=True):
+        assert torch.equal(b[0], K[..., s:e, :]) and torch.equal(b[1], V[..., s:e, :])
+
+
+def test_extract_host_tables_refuse_bad_spans():
+    """The host-table entry checks spans, alignment and count before any launch."""
+    L, H, N, D = 2, 2, 40, 64
+    K = torch.zeros((L, 1, H, N, D), dtype=torch.bfloat16, device=DEV)
+    dst = torch.zeros((2, L, 1, H, 11, D), dtype=torch.bfloat16, device=DEV)
+    call = lambda at, n, start, ln: _native.lib().ckv_extract_chunks_host(
+        K.data_ptr(), K.data_ptr(), H * N * D, N * D, (ctypes.c_uint64 * n)(*[at] * n),
+        (ctypes.c_int32 * (2 * n))(*[start, ln] * n), n, L, H, N, D, _native.DTYPE_BF16,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    codes = [call(dst.data_ptr(), 1, 30, 11), call(dst.data_ptr(), 1, -1, 2), call(dst.data_ptr() + 8, 1, 0, 11),
+             call(dst.data_ptr(), 65, 0, 11)]
+    assert all(c != 0 for c in codes), codes
+    assert codes[0] == codes[1] and len(set(codes)) == 3
