@@ -108,12 +108,20 @@ void check(int32_t status, const char* what) {
   if (status == CKV_ERR_INVALID_ARGUMENT || status == CKV_ERR_OUT_OF_RANGE || status == CKV_ERR_TOO_LARGE) value_error(msg);
   throw PyFailure{PyExc_RuntimeError, msg};
 }
-// The launch itself runs without the interpreter lock, as a ctypes call does.
+// The launch itself runs without the interpreter lock, as a ctypes call does. f looks up addresses
+// and the stream too, which throw (a tensor without storage, a HIP error): the lock is taken back
+// on that way out as well, before any handler touches the interpreter.
+struct Unlocked {
+  PyThreadState* const state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
 template <typename F>
 int32_t unlocked(F f) {
-  int32_t r;
-  Py_BEGIN_ALLOW_THREADS r = f();
-  Py_END_ALLOW_THREADS return r;
+  const Unlocked section;
+  return f();
 }
 
 // attention_active(q, K, V, positions, scale, err, out, split)
