@@ -34,21 +34,13 @@
 // eight wavefronts on one tile (233 / 476), 48 or 64 queries a wavefront (275 / 453, 322 / 649).
 #include <algorithm>
 
+#include "attention_plan.hpp"
 #include "ckv_common.hpp"
 
 namespace ckv {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-#ifndef CKV_ATTN_QG
-#define CKV_ATTN_QG 2
-#endif
-constexpr int kAttnWaves = 4;
-constexpr int kAttnQG = CKV_ATTN_QG;                // 16-query groups per wavefront
-constexpr int kAttnBM = kAttnWaves * kAttnQG * 16;  // queries per workgroup
-constexpr int kAttnBN = 64;                         // cache rows per tile
-constexpr int kWaveChunk = 32;                      // cache rows per step of attn_wave_kernel's wavefronts
 
 // Combine a lane's value with the lanes 16 and 32 away (the four lane groups of one query), with
 // gfx950's row-swap permutes (VALU, no LDS round trip): each returns the lane's own value and
@@ -113,33 +105,10 @@ __device__ __forceinline__ bf16x8 v_operand(const char* vb, int dt, int g, int l
   return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-constexpr int kXcds = 8;  // MI355X: workgroups go round-robin to 8 XCDs, each with its own L2
-
-// Which work item (query block qb, head h, cache split z) a workgroup takes. The hardware hands
-// workgroup L of a 1-D grid to XCD L % 8, so items are assigned through L: the XCDs split evenly
-// over the KV heads (8 / Hkv XCDs each), every item of one KV head lands on that head's XCDs (its
-// K/V stay in their L2s and are read there by all `group` query heads together), consecutive items
-// of an XCD cycle through the group's query heads on one query block and split, and query blocks
-// go latest position first, alternating between the head's XCDs so their work stays balanced. The
-// grid is padded to whole rounds of 8; a workgroup past a head's last item returns. With a KV-head
-// count that does not divide 8, all heads are one group over all XCDs. The two divisions are
-// multiplications by the host's reciprocals: hardware has no integer division, and four or five
-// emulated ones were half a microsecond of every workgroup's start.
-struct AttnMap {
-  int nqb = 0, group = 0, xpk_log = 0, items = 0;  // items: of one KV head
-  uint32_t inv_group = 0, inv_nqb = 0;
-  dim3 grid;
-};
-
-// x / d for d > 0: through inv = ceil(2^32 / d) where the host found that exact for every x here
-// (x d < 2^32), 0 elsewhere.
+// x / d for d > 0, with inv = inverse_of(.., d).
 __device__ __forceinline__ int div_by(int x, int d, uint32_t inv) {
   return inv != 0 ? (int)__umulhi((uint32_t)x, inv) : d == 1 ? x : x / d;
 }
-static uint32_t inverse_of(int64_t most, int64_t d) {  // for x <= most
-  return d > 1 && most * d < (1ll << 32) ? (uint32_t)(((1ll << 32) + d - 1) / d) : 0;
-}
-
 __device__ __forceinline__ bool attn_work_item(int nqb, int group, int xpk_log, int items, uint32_t inv_group,
                                                uint32_t inv_nqb, int& qb, int& h, int& z) {
   const int L = (int)blockIdx.x, xcd = L % kXcds;
@@ -149,22 +118,6 @@ __device__ __forceinline__ bool attn_work_item(int nqb, int group, int xpk_log, 
   z = div_by(rest, nqb, inv_nqb);
   qb = nqb - 1 - (rest - z * nqb);
   return j < items;
-}
-
-static AttnMap attn_map(int64_t nqb, int Hkv, int group, int64_t splits) {
-  AttnMap m;
-  if (kXcds % Hkv != 0) {
-    group *= Hkv;
-    Hkv = 1;
-  }
-  while ((Hkv << m.xpk_log) < kXcds) ++m.xpk_log;
-  m.nqb = (int)nqb;
-  m.group = group;
-  m.items = (int)(group * nqb * splits);
-  m.inv_group = inverse_of(m.items, group);
-  m.inv_nqb = inverse_of(nqb * splits, nqb);
-  m.grid = dim3((unsigned)((((int64_t)m.items + (1 << m.xpk_log) - 1) >> m.xpk_log) * kXcds));
-  return m;
 }
 
 template <int D>
@@ -428,96 +381,15 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
 
 #include "attention_wave.hpp"
 
-namespace ckv {
-
-// How a launch runs.
-struct AttnPlan {
-  bool wave = false;     // attn_wave_kernel, else attn_active_kernel
-  bool grouped = false;  // rows are the (token, query head) pairs of a KV head
-  int qg = 0, waves = 0;
-  int splits = 1, split_chunks = 0;
-  AttnMap map;
-};
-
-// The (head_dim, QG, W, GROUPED) forms of attn_wave_kernel that attn_plan picks from.
-#define CKV_WAVE_FORMS(X)                                                                  \
-  X(128, 1, 4, true) X(128, 1, 8, true) X(128, 2, 8, true)                                  \
-  X(128, 1, 4, false) X(128, 1, 8, false) X(128, 2, 4, false) X(128, 2, 8, false)           \
-  X(64, 1, 4, true) X(64, 1, 8, true)                                                       \
-  X(64, 1, 4, false) X(64, 1, 8, false) X(64, 2, 4, false) X(64, 2, 8, false)
-
-// Where the 128-query workgroups are too few: below about one for each of the 256 CUs at head_dim
-// 128 (us, 28 heads, this first: 768 causal rows, 168 workgroups, 19.7 against 20.6; 1000 of 8256
-// rows, 224, 157 against 164; 1103 causal rows, 252, 27.8 against 27.1; 1500, 336, 41.1 against
-// 36.5), below two at head_dim 64, where they also hold less work each (14 heads: 3000 causal rows,
-// 336 workgroups, 37.6 against 46.5; 4000, 448, 58.9 against 61.8; 4500, 504, 72.4 against 69.8).
-static bool wave_launch(int n, int Hq, int head_dim) {
-  const int64_t blocks = (int64_t)((n + kAttnBM - 1) / kAttnBM) * Hq;
-  return blocks < (head_dim == 128 ? 256 : 450);
-}
-
-constexpr int kWaveFill = 256;  // workgroups that a split launch aims at: one for each CU
-
-// The most splits a launch takes: a workgroup has at most 32 (token, query head) rows, a split's
-// four wavefronts a chunk each.
-static int64_t most_splits(int n, int N, int Hq, int head_dim) {
-  const int64_t chunks = (N + kWaveChunk - 1) / kWaveChunk;
-  if (!wave_launch(n, Hq, head_dim) || chunks <= 16) return 1;
-  return std::max<int64_t>(1, std::min<int64_t>(kWaveFill * 32 / ((int64_t)n * Hq), (chunks + 3) / 4));
-}
-
-static AttnPlan attn_plan(int n, int N, int Hq, int Hkv, int head_dim, int64_t workspace_bytes) {
-  AttnPlan p;
-  const int group = Hq / Hkv;
-  if (!wave_launch(n, Hq, head_dim)) {
-    p.map = attn_map((n + kAttnBM - 1) / kAttnBM, Hkv, group, 1);
-    return p;
-  }
-  p.wave = true;
-  p.grouped = group > 1 && (int64_t)n * group <= kAttnBM;
-  const int rows = p.grouped ? n * group : n, heads = p.grouped ? Hkv : Hq;
-  const int chunks = (N + kWaveChunk - 1) / kWaveChunk;
-  const int b16 = (rows + 15) / 16 * heads, b32 = (rows + 31) / 32 * heads;
-  // 16 rows a workgroup while those workgroups are all resident at once (two or four of four
-  // wavefronts on a CU, by registers), else 32, which read each cache row half as often: 28 heads
-  // of 128, 192 causal rows 5.9 against 7.2 us, 320 rows (560 workgroups) 9.8 against 9.0. A long
-  // cache is read often enough to prefer 32 earlier at head_dim 128 (251 of 1103 rows 13.7 against
-  // 14.1, 300 of 4000 34 against 43).
-  const bool lng = chunks >= 24;
-  if (rows <= 16) p.qg = 1;
-  else if (lng) p.qg = head_dim == 64 && b16 <= 512 ? 1 : 2;
-  else p.qg = b16 <= (head_dim == 64 ? 800 : 512) ? 1 : 2;
-  const int blocks = p.qg == 1 ? b16 : b32;
-  // Eight wavefronts halve a workgroup's chain where it is long, if the workgroups still fit (one
-  // or two on a CU): 300 of 4000 rows 34 against 45 us with four, 768 causal rows 24.5 against 19.1.
-  p.waves = lng && (blocks <= 288 || (blocks <= 450 && chunks >= 128)) ? 8 : 4;
-  // Splits cost the merge launch, about 3 us: taken for one token's rows from 17 chunks on (28
-  // heads, 700 rows 7.1 against 8.5 us, 8288 rows 8.7 against 45), else where eight wavefronts
-  // would have eight chunks each (150 of 1500 rows, 47 chunks, 8.5 us whole and 9.5 in two).
-  int64_t splits = std::min<int64_t>(most_splits(n, N, Hq, head_dim), kWaveFill / std::max(blocks, 1));
-  if (rows > 16 && chunks < 64) splits = 1;
-  const int64_t row_b = (int64_t)Hq * n * (head_dim + 4) * 4;
-  splits = std::min<int64_t>(splits, workspace_bytes / row_b);
-  if (rows <= 16) p.waves = splits > 1 ? 4 : 8;
-  splits = std::max<int64_t>(1, std::min<int64_t>(splits, (chunks + p.waves - 1) / p.waves));
-  p.split_chunks = (int)((chunks + splits - 1) / splits);
-  p.splits = (chunks + p.split_chunks - 1) / p.split_chunks;
-  p.map = attn_map(blocks / heads, Hkv, p.grouped ? 1 : group, p.splits);
-  return p;
-}
-
-}  // namespace ckv
-
 extern "C" int64_t ckv_attention_workspace_bytes(int32_t n_queries, int32_t n_tokens, int32_t n_q_heads,
                                                  int32_t head_dim, int32_t* splits_out, int32_t* split_tiles_out) {
   using namespace ckv;
-  int64_t splits = 1;
-  if (n_queries > 0 && n_tokens > 0 && n_q_heads > 0 && head_dim > 0)
-    splits = most_splits(n_queries, n_tokens, n_q_heads, head_dim);
+  const bool some = n_queries > 0 && n_tokens > 0 && n_q_heads > 0 && head_dim > 0;
+  const int64_t splits = some ? most_splits(n_queries, n_tokens, n_q_heads, head_dim) : 1;
   const int tiles = n_tokens > 0 ? (n_tokens + kAttnBN - 1) / kAttnBN : 0;
   if (splits_out != nullptr) *splits_out = (int32_t)splits;
   if (split_tiles_out != nullptr) *split_tiles_out = splits > 1 ? (int32_t)((tiles + splits - 1) / splits) : 0;
-  return splits > 1 ? splits * n_q_heads * n_queries * (head_dim + 4) * 4 : 0;
+  return some ? attn_workspace_bytes(n_queries, n_tokens, n_q_heads, head_dim) : 0;
 }
 
 extern "C" int32_t ckv_attention_active(void* out, const void* q, int64_t q_head_stride, int64_t q_token_stride,
@@ -546,7 +418,7 @@ extern "C" int32_t ckv_attention_active(void* out, const void* q, int64_t q_head
   const AttnMap& map = plan.map;
   if (!plan.wave) {
     auto launch = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, map.grid, dim3(kAttnWaves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
+      hipLaunchKernelGGL(kernel, dim3(map.blocks), dim3(kAttnWaves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
                          map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
                          (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
                          n_q_heads, group, scale_log2, (char*)out, err);
@@ -559,7 +431,7 @@ extern "C" int32_t ckv_attention_active(void* out, const void* q, int64_t q_head
   float* ws = plan.splits > 1 ? (float*)workspace : nullptr;
   const uint32_t inv_gqa = inverse_of((int64_t)n_queries * group, group);
   auto launch = [&](auto kernel, int waves) {
-    hipLaunchKernelGGL(kernel, map.grid, dim3(waves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
+    hipLaunchKernelGGL(kernel, dim3(map.blocks), dim3(waves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
                        map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
                        (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
                        n_q_heads, group, inv_gqa, scale_log2, plan.split_chunks, (char*)out, ws, err);

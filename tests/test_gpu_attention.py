@@ -153,3 +153,18 @@ def test_attention_small_launch_forms(Hq, Hkv, D, N, n):
         K[:, seen:], V[:, seen:] = 0, 0
         out, _ = _run(q, K, V, pos)
         np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,N,n", [
+    (130, 65, 64, 768, 57),   # 114 grouped rows, long cache
+    (130, 65, 128, 300, 64),  # 128 grouped rows, short cache
+    (146, 73, 128, 1000, 57),
+    (160, 80, 64, 40, 50),
+])
+def test_attention_more_kv_heads_than_a_grouped_launch_fills(Hq, Hkv, D, N, n):
+    """More than 64 KV heads, whose grouped launches run the nearest form there is. Tolerance as at
+    the top of this file."""
+    q, K, V, pos = _case(Hq + n, Hq, Hkv, D, N, n)
+    out, e = _run(q, K, V, pos)
+    assert e == 0
+    np.testing.assert_allclose(out[0].float().cpu().numpy(), O.attention_active(q, K, V, pos), atol=ATOL, rtol=0)
