@@ -9,6 +9,7 @@
 // host for each: attention_active 9.4 us, rope_qkv (k/v into a cache) 10.9, add_rmsnorm 8.0,
 // silu_mul 12.2. The launch itself is 2-3 us of that.
 #include <Python.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -325,6 +326,17 @@ PyObject* silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   CKV_PY_END
 }
 
+// Whether a call with these operands would reach torch's device code with nothing in between: no
+// tracing, transform (vmap), mode, autocast or tensor subclass takes part, which the kernels here
+// know nothing of.
+bool unintercepted(c10::DispatchKeySet operands) {
+  static const c10::DispatchKeySet plain({c10::DispatchKey::CUDA, c10::DispatchKey::AutogradCUDA,
+                                          c10::DispatchKey::ADInplaceOrView, c10::DispatchKey::BackendSelect});
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  const c10::DispatchKeySet keys = (operands | tls.included_) - tls.excluded_;
+  return (keys.raw_repr() & ~plain.raw_repr()) == 0;
+}
+
 // linear(x, weight, bias): ckv_linear where it is the better choice and takes the operands, else torch's
 PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   CKV_PY_BEGIN
@@ -332,7 +344,8 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t n_args) {
   const Tensor &x = tensor(a[0]), &w = tensor(a[1]), bias = optional_tensor(a[2]);
   auto plain = [&](const Tensor& t) {
     return t.is_cuda() && t.device() == x.device() && t.scalar_type() == at::kBFloat16 && t.is_contiguous() &&
-           (uintptr_t)t.data_ptr() % 16 == 0 && !(at::GradMode::is_enabled() && t.requires_grad());
+           unintercepted(t.key_set()) && !t._fw_grad(/*level=*/0).defined() && (uintptr_t)t.data_ptr() % 16 == 0 &&
+           !(at::GradMode::is_enabled() && t.requires_grad());
   };
   int64_t ws_bytes = -1;
   if (x.dim() >= 2 && w.dim() == 2 && x.size(-1) == w.size(1) && w.numel() > 0 && x.numel() > 0 && plain(x) && plain(w) &&

@@ -133,13 +133,17 @@ def _stack_params(mods: list, name: str) -> torch.Tensor | None:
     return stacked
 
 
+_LINEAR_FORWARD = torch.nn.Linear.forward
+
+
 def _apply_linear(m, x: torch.Tensor) -> torch.Tensor:
-    """m(x); for an nn.Linear that nothing wraps, hooks or patches, its product by ops.linear."""
-    if (type(m) is torch.nn.Linear and not m._forward_hooks and not m._forward_pre_hooks
-            and "forward" not in m.__dict__ and not torch.nn.modules.module._has_any_global_hook()):
-        w = m._parameters.get("weight")
-        if w is not None:
-            return ops.linear(x, w, m._parameters.get("bias"))
+    """m(x); for an nn.Linear that nothing wraps, hooks, compiles or patches, its product by ops.linear."""
+    p = m._parameters
+    if (type(m) is torch.nn.Linear and torch.nn.Linear.forward is _LINEAR_FORWARD and "forward" not in m.__dict__
+            and m._compiled_call_impl is None and "weight" in p and "bias" in p
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and not torch.nn.modules.module._has_any_global_hook()):
+        return ops.linear(x, p["weight"], p["bias"])
     return m(x)
 
 

@@ -12,6 +12,8 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
+import torch.nn.functional as F
+from torch.overrides import has_torch_function_variadic
 
 from chunkkv_amd import _native
 from chunkkv_amd._native import check, lib
@@ -711,5 +713,8 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
 
 def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
     """torch.nn.functional.linear(x, weight, bias): on ckv_linear for the bf16 projections of short
-    requests (contiguous operands, no gradient asked for), on torch's library call for the rest."""
+    requests (contiguous operands, no gradient or tangent asked for, nothing between the call and the
+    device: no autocast, transform, mode or tensor subclass), on torch's own call for the rest."""
+    if has_torch_function_variadic(x, weight, bias):
+        return F.linear(x, weight, bias)
     return _native.torch_ops().linear(x, weight, bias)

@@ -91,3 +91,22 @@ def test_linear_keeps_gradients_and_wrapped_modules():
         m.register_forward_hook(lambda *a: seen.append(1))
         _apply_linear(m, x)
         assert seen == [1]
+
+
+def test_linear_under_transforms_equals_torch():
+    """Autocast of another type, vmap, forward-mode tangents: as torch's own call, at a size that
+    ckv_linear takes without them."""
+    import torch.autograd.forward_ad as fw
+
+    x, w, b = _operands(10, 64, 64)
+    with torch.autocast("cuda", torch.float16):
+        y = ops.linear(x, w, b)
+        assert y.dtype == torch.float16 and torch.equal(y, F.linear(x, w, b))
+    with torch.autocast("cuda", torch.bfloat16):
+        assert torch.equal(ops.linear(x.float(), w, b), F.linear(x.float(), w, b))
+    xs = torch.stack([x[0], -x[0]])
+    assert torch.equal(torch.func.vmap(lambda a: ops.linear(a, w, b))(xs), torch.func.vmap(lambda a: F.linear(a, w, b))(xs))
+    with fw.dual_level():
+        d = fw.make_dual(x, x.flip(1))
+        got, want = (fw.unpack_dual(f(d, w, b)) for f in (ops.linear, F.linear))
+        assert torch.equal(got.primal, want.primal) and torch.equal(got.tangent, want.tangent)

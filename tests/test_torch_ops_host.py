@@ -68,3 +68,62 @@ with FakeTensorMode():
     assert [line[0] for line in lines] == want
     # torch computes a product of fake tensors as a fake tensor: linear may return one
     assert all(line[1] == "raised" or line[0] == "linear" for line in lines), out
+
+
+def test_linear_leaves_transforms_modes_and_subclasses_to_torch():
+    """Products that ckv_linear would take by type and shape, on fake tensors: whatever sits between a
+    call and the device takes part as in torch.nn.functional.linear."""
+    out = _child("""
+import torch.autograd.forward_ad as fw
+from torch.overrides import TorchFunctionMode
+seen = []
+class Functions(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        seen.append(func.__name__)
+        return func(*args, **(kwargs or {}))
+class Wrapped(torch.Tensor):
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        seen.append(func.__name__)
+        return "wrapped"
+with FakeTensorMode():
+    x, w = t(10, 64), t(64, 64)
+    y = ops.linear(x, w)
+    assert type(y).__name__ == "FakeTensor" and y.shape == (10, 64) and y.dtype == BF
+    y = batched(lambda a: ops.linear(a, w), x)
+    assert y.shape == (2, 10, 64)
+    with fw.dual_level():
+        for args in ((fw.make_dual(x, t(10, 64)), w), (x, fw.make_dual(w, t(64, 64))), (x, w, fw.make_dual(t(64), t(64)))):
+            assert fw.unpack_dual(ops.linear(*args)).tangent is not None
+    with Functions():
+        ops.linear(x, w)
+    assert seen == ["linear"], seen
+assert ops.linear(torch.zeros(4, 64).as_subclass(Wrapped), torch.zeros(64, 64)) == "wrapped"
+print("ok")
+""")
+    assert out.strip() == "ok"
+
+
+def test_apply_linear_calls_what_is_not_a_plain_linear(monkeypatch):
+    """HipEngine's shortcut past nn.Linear.__call__ is taken for nothing that changes what the call
+    does."""
+    import torch
+
+    from chunkkv_amd import engine, ops
+
+    monkeypatch.setattr(ops, "linear", lambda *a: "shortcut")
+    x, made = torch.zeros(2, 8), lambda: torch.nn.Linear(8, 8)
+    assert engine._apply_linear(made(), x) == "shortcut"
+
+    hooked, compiled, replaced, moved = made(), made(), made(), made()
+    hooked.register_forward_hook(lambda *a: "hook")
+    compiled._compiled_call_impl = lambda *a: "compiled"
+    replaced.forward = lambda *a: "forward"
+    bias = moved._parameters.pop("bias").detach()
+    moved.bias = bias + 1.0
+    assert engine._apply_linear(hooked, x) == "hook"
+    assert engine._apply_linear(compiled, x) == "compiled"
+    assert engine._apply_linear(replaced, x) == "forward"
+    assert torch.equal(engine._apply_linear(moved, x), (bias + 1.0).expand(2, 8))
+    monkeypatch.setattr(torch.nn.Linear, "forward", lambda *a: "class")
+    assert engine._apply_linear(made(), x) == "class"
