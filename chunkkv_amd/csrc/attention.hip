@@ -214,13 +214,14 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   // Tile loads go straight from global memory to LDS (global_load_lds_dwordx4): load
   // instruction i of wavefront w fills the 1 KB block w * KI + i of a tile buffer, lane l its 16
   // bytes at l * 16, i.e. position P = (w KI + i) 64 + l = slot P / CPR, chunk P % CPR. No
-  // registers stage the tile and no LDS store instructions run; rows past the cache load row
-  // N - 1 instead (every query's position is below them, so they are masked).
+  // registers stage the tile and no LDS store instructions run; rows past every query's position
+  // load the last one's row instead: they are masked, but their zero weights meet the values, and a
+  // cache row not written yet may hold a NaN (nor is there a row past the cache to read).
   constexpr int KI = (kAttnBN * CPR) / NT;  // load instructions per wavefront, tile and tensor
   static_assert(KI >= 1 && (kAttnBN * CPR) % NT == 0, "a tile must fill whole load instructions");
   // A lane's offsets in a tile are kept (K slots hold rows in kslot_row's order) and added to the
   // tile's uniform address: two 64-bit addresses built per load were a quarter of a tile's vector
-  // instructions. Only a tile that reaches past the cache clamps its rows.
+  // instructions. Only a workgroup's last tile clamps its rows.
   int off_k[KI], off_v[KI];
 #pragma unroll
   for (int i = 0; i < KI; ++i) {
@@ -234,7 +235,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   auto issue = [&](int n0, char* kb, char* vb) {
     const char* kt = kh + (int64_t)n0 * ROWB;
     const char* vt = vh + (int64_t)n0 * ROWB;
-    const int last = N - 1 - n0;  // >= 0: only tiles that some query sees are issued
+    const int last = bmax - n0;  // >= 0: only tiles that some query sees are issued
     auto load = [&](const char* t, int off, char* to) {
       __builtin_amdgcn_global_load_lds((gvoid*)(t + (uint32_t)off), (lvoid*)to, 16, 0, 0);
     };

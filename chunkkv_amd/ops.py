@@ -626,8 +626,9 @@ def attention_active(
     """Attention of the active query rows over the cache, query i seeing positions <= positions[i]
     (the reference's boolean-mask SDPA with enable_gqa, torch_engine.py:157 and :68-72).
 
-    q: (1, Hq, n, D) bf16 with contiguous rows; K/V: (1, Hkv, N, D) contiguous; positions: int64
-    (n,). Returns (1, n, Hq, D) bf16, token-major (``.view(1, n, Hq * D)`` feeds o_proj).
+    q: (1, Hq, n, D) bf16 with contiguous rows; K/V: (1, Hkv, N, D) contiguous, their rows past the
+    largest position anything, not written yet too; positions: int64 (n,). Returns (1, n, Hq, D)
+    bf16, token-major (``.view(1, n, Hq * D)`` feeds o_proj).
     split: let launches too small to fill the chip split the cache range (a workspace is
     allocated for the partial results).
     """

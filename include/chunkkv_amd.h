@@ -520,7 +520,8 @@ int32_t ckv_extract_chunks_host(const void* k_slab, const void* v_slab, int64_t 
  *   q          bf16 (n_q_heads, n_queries, head_dim) with the given head/token strides (elements,
  *              multiples of 8; rows contiguous)
  *   k_cache,   bf16 (n_kv_heads, n_tokens, head_dim), rows contiguous, head stride kv_head_stride
- *   v_cache
+ *   v_cache    of at least n_tokens * head_dim; rows past the largest position may hold anything,
+ *              NaN too, rows up to it are finite
  *   positions  int64 (n_queries,), each in [0, n_tokens) (out-of-range entries are clamped and
  *              flagged in *err); any order, ascending is fastest
  *   out        bf16 (n_queries, n_q_heads, head_dim) contiguous: token-major, the layout the

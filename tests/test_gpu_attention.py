@@ -132,11 +132,14 @@ def test_attention_split_launch_matches_oracle_and_unsplit(Hq, Hkv, D, N, n):
     (28, 4, 128, 1180, 1152),  # 252 128-query workgroups: the last size below the large kernel's range
     (28, 4, 128, 1181, 1153),  # 280: the first inside it
     (16, 16, 64, 2100, 40),  # no grouping, split
+    (28, 4, 128, 1408, 1280),  # the large kernel, its last tile three rows past the positions
+    (8, 8, 64, 7990, 7950),  # the same at head_dim 64, the last tile also past the cache
 ])
 def test_attention_small_launch_forms(Hq, Hkv, D, N, n):
     """Every form of the small-launch kernel (rows and wavefronts per workgroup, grouped rows, splits)
-    at the edges of its range: against the oracle, unsplit, and with the rows past every position
-    uninitialised (NaN), which no query may see. Tolerance as at the top of this file."""
+    at the edges of its range, and the large kernel beyond: against the oracle, unsplit, and with the
+    rows past every position uninitialised (NaN), which no query may see. Tolerance as at the top of
+    this file."""
     q, K, V, pos = _case(N * 7 + n, Hq, Hkv, D, N, n)
     seen = max(1, N - 3)
     pos = np.minimum(pos, seen - 1)
@@ -146,12 +149,7 @@ def test_attention_small_launch_forms(Hq, Hkv, D, N, n):
     whole = ops.attention_active(*args, split=False)
     sub = np.unique(np.linspace(0, n - 1, min(n, 200)).astype(int))
     want = O.attention_active(q[:, sub], K[:, :seen], V[:, :seen], pos[sub])
-    small = -(-n // 128) * Hq < (256 if D == 128 else 450)
-    for out in (got, whole) if small else ():
-        np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
-    if not small:  # the large kernel multiplies zero weights into the rest of its last tile
-        K[:, seen:], V[:, seen:] = 0, 0
-        out, _ = _run(q, K, V, pos)
+    for out in (got, whole):
         np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
 
 
