@@ -22,6 +22,15 @@
 
 namespace ckv {
 
+// Between the stages in which a wavefront's lanes exchange rows through LDS (and before a stage's rows
+// are overwritten): LDS runs one wavefront's operations in order, so this is no instruction, only an
+// order of stores and loads that the compiler has to keep though no lane reads its own bytes.
+__device__ __forceinline__ void wave_lds_stage() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 template <int D, int QG, int W, bool GROUPED>
 __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
     int nqb, int map_group, int xpk_log, int items, uint32_t inv_group, uint32_t inv_nqb,
@@ -87,6 +96,7 @@ __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
   bf16x8 qf[QG][DS];
 #pragma unroll
   for (int i = 0; i < QI; ++i) put((i * 64 + lane) / CPR, qr[i]);
+  wave_lds_stage();
 #pragma unroll
   for (int qg = 0; qg < QG; ++qg)
 #pragma unroll
@@ -124,12 +134,14 @@ __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
   }
   for (; c < c_end; c += W) {
     const int n0 = c * kWaveChunk;
+    wave_lds_stage();
 #pragma unroll
     for (int i = 0; i < LI; ++i) {  // K row r = 8 a + 4 t + b to slot 16 t + 4 a + b (kslot_row's inverse)
       const int r = (i * 64 + lane) / CPR;
       put(16 * ((r >> 2) & 1) + 4 * (r >> 3) + (r & 3), kr[i]);
     }
     if (c + W < c_end) load(kr, kh, c + W);  // lands while this chunk is worked on
+    wave_lds_stage();
     f32x4 s[QG][2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -143,6 +155,7 @@ __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
     // V over the K rows; rows past every query's position become zero (their weights are zero, and
     // a cache row not written yet may hold a NaN)
     const bool edge = n0 + kWaveChunk - 1 > wmax;
+    wave_lds_stage();
 #pragma unroll
     for (int i = 0; i < LI; ++i) {
       const int slot = (i * 64 + lane) / CPR;
@@ -150,6 +163,7 @@ __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
       *(vec16*)(wl + slot * ROWB + (((lane % CPR) ^ swz_v<CPR>(slot)) * 16)) = v;
     }
     if (c + W < c_end) load(vr, vh, c + W);
+    wave_lds_stage();
 
     const bool need_mask = n0 + kWaveChunk - 1 > wmin;
     bf16x8 pb[QG];
