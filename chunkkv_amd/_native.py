@@ -17,7 +17,7 @@ import torch  # noqa: F401  (must precede the CDLL load, see module docstring)
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libchunkkv_amd.so"
 TORCH_OPS_PATH = LIB_PATH.with_name("_torch_ops.so")
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 CKV_OK = 0
 CKV_ERR_INVALID_ARGUMENT = 1
@@ -149,13 +149,14 @@ def lib() -> ctypes.CDLL:
                 f"{LIB_PATH} is not built; run `python -m chunkkv_amd.build` (there is no CPU fallback)"
             )
         handle = ctypes.CDLL(str(LIB_PATH), mode=os.RTLD_NOW | os.RTLD_LOCAL)
+        # the version before the signatures: an older library may lack some of them
+        ver = handle.ckv_abi_version()
+        if ver != ABI_VERSION:
+            raise NativeLibraryMissing(f"{LIB_PATH} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")
         for name, (res, args) in SIGNATURES.items():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-        ver = handle.ckv_abi_version()
-        if ver != ABI_VERSION:
-            raise NativeLibraryMissing(f"{LIB_PATH} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")
         _lib = handle
     return _lib
 

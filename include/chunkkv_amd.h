@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define CKV_ABI_VERSION 5
+#define CKV_ABI_VERSION 6
 
 typedef enum ckv_status {
   CKV_OK = 0,

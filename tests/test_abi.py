@@ -36,6 +36,18 @@ def test_library_loads_and_exports_every_declared_symbol():
     assert set(names) <= exported
 
 
+def test_an_older_library_is_named_by_its_version(tmp_path, monkeypatch):
+    """A library of another ABI version, without entry points that were added since: the error says
+    which version it is, not which symbol it lacks."""
+    src, so = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text(f"int ckv_abi_version(void) {{ return {_native.ABI_VERSION - 1}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    monkeypatch.setattr(_native, "LIB_PATH", so)
+    monkeypatch.setattr(_native, "_lib", None)
+    with pytest.raises(_native.NativeLibraryMissing, match=f"ABI version {_native.ABI_VERSION - 1}, expected {_native.ABI_VERSION}"):
+        _native.lib()
+
+
 def test_status_strings():
     lib = _native.lib()
     assert lib.ckv_status_string(0) == b"ok"
