@@ -182,7 +182,7 @@ class HipEngine(DecoderPieces):
         self._init_model(model, tokenizer)
         if self.device.type != "cuda":
             raise ValueError("HipEngine runs on a HIP device: move the model to 'cuda' first")
-        _native.lib()  # raises now if the kernels were never built: there is no CPU fallback
+        _native.torch_ops()  # raises now if the kernels or their calls were never built: there is no CPU fallback
         self.kv_dtype = self.layers[0].self_attn.k_proj.weight.dtype
         ops.dtype_code(self.kv_dtype)
         self.inv_freq = ops.inv_freq(self.head_dim, self.theta, self.device)

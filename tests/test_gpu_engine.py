@@ -485,3 +485,13 @@ def test_chunk_address_memo_follows_replaced_layers(models, parts):
     third = eng.prefill(toks2, pl, cfg)
     assert not torch.equal(first.keys[2], second.keys[2])
     assert torch.equal(first.keys[2], third.keys[2]) and torch.equal(first.logits, third.logits)
+
+
+def test_engine_needs_the_native_calls(models, tmp_path, monkeypatch):
+    """Without the native per-layer calls construction raises, not the first prefill."""
+    from chunkkv_amd import _native
+
+    monkeypatch.setattr(_native, "_ops", None)
+    monkeypatch.setattr(_native, "TORCH_OPS_PATH", tmp_path / "_torch_ops.so")
+    with pytest.raises(_native.NativeLibraryMissing, match="not built"):
+        HipEngine(models[1], StubTokenizer())
