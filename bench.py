@@ -856,18 +856,17 @@ def bench_deviation_topk(steps: int, warmup: int, dev) -> dict:
     return line
 
 
-# Four HipEngine prefills in flight, one host thread each (bench_replay's concurrent TTFT), stopped
-# making progress in two of three runs on the GPU (no output for 3 minutes, the run killed) after
-# completing in the others at 448-520 ms p50. No kernel of this library waits for another
-# workgroup or launch, and no host path of the engine waits across streams without overlap, so the
-# stall lies in what the four threads share (the library GEMMs' kernels and the HIP runtime); its
-# cause is not found. The measurement runs only when asked for (--concurrent-ttft).
-CONCURRENT_TTFT_NOTE = ("4 concurrent 32k prefills (one host thread each) not measured by default: runs of it "
-                        "stalled with no progress on the GPU, cause not found; --concurrent-ttft runs it")
+# Four HipEngine prefills in flight, one host thread each (config 5's concurrent TTFT), stopped making
+# progress in two of three runs on the GPU (no output for 3 minutes, the run killed) after completing
+# in the others at 448-520 ms p50. No kernel of this library waits for another workgroup or launch,
+# and no host path of the engine waits across streams without overlap, so the stall lies in what the
+# four threads share (the library GEMMs' kernels and the HIP runtime); its cause is not found. Until it
+# is, the measurement is switched off: --concurrent-ttft is an error.
+CONCURRENT_TTFT_NOTE = ("4 concurrent 32k prefills (one host thread each) not measured: runs of it stalled with no "
+                        "progress on the GPU, cause not found")
 
 
-def bench_replay(steps: int, warmup: int, dev, n_streams: int = 4, ttft_requests: int = 6, model=None,
-                 concurrent_ttft: bool = False) -> dict:
+def bench_replay(steps: int, warmup: int, dev, n_streams: int = 4, ttft_requests: int = 6, model=None) -> dict:
     """Long-context multi-request replay at the Qwen2.5-7B shape: an HBM-resident store of 256
     chunks x 256 tokens x 2 context variants (7.0 GiB); 4 concurrent requests of 128 chunks
     sampled with replacement (Zipf s=1.1) at random order + a 64-token query (32832 tokens), 15%
@@ -879,8 +878,7 @@ def bench_replay(steps: int, warmup: int, dev, n_streams: int = 4, ttft_requests
     follow the cached ones (per-chunk noise) and again with uncorrelated random rows (the
     selection's hardest input). Then TTFT p50/p99 of HipEngine.prefill + last_logprobs on requests
     of the same shape (random-init Qwen2.5-7B architecture, bf16; the store's K/V serve as the
-    cached chunks), one at a time, and with concurrent_ttft also with 4 requests in flight, each
-    from its own host thread (off by default: see CONCURRENT_TTFT_NOTE)."""
+    cached chunks), one at a time (CONCURRENT_TTFT_NOTE says why not several at once)."""
     from chunkkv_amd import ops
     from chunkkv_amd.planner import local_index, plan_request
 
@@ -1037,74 +1035,12 @@ def bench_replay(steps: int, warmup: int, dev, n_streams: int = 4, ttft_requests
         line["ttft_note"] = ("HipEngine; ttft_p50_ms / ttft_p99_ms one request at a time; the reference op "
                              "sequence is not timed at 32k (its math-path SDPA would hold ~120 GB of fp32 scores "
                              "per layer)")
-        if concurrent_ttft:
-            conc = _concurrent_ttft(model, cfg, placements_of, n_streams, max(ttft_requests, 20), N, vocab, dev)
-            line["ttft_p50_ms_concurrent"] = round(float(np.percentile(conc, 50)), 2)
-            line["ttft_p99_ms_concurrent"] = round(float(np.percentile(conc, 99)), 2)
-            line["ttft_requests_concurrent"] = len(conc)
-            line["ttft_note"] += (f"; *_concurrent with {n_streams} requests in flight (one host thread, HipEngine "
-                                  "and HIP stream per request, each request's prefill + last_logprobs timed from "
-                                  "the round's start)")
-        else:
-            line["ttft_concurrent_note"] = CONCURRENT_TTFT_NOTE
+        line["ttft_concurrent_note"] = CONCURRENT_TTFT_NOTE
         del hip
         if own_model:
             del model
         torch.cuda.empty_cache()
     return line
-
-
-def _concurrent_ttft(model, cfg, placements_of, n_streams: int, rounds: int, N: int, vocab: int, dev) -> list:
-    """TTFT (ms) of `rounds` rounds of n_streams concurrent HipEngine prefills + last_logprobs, one
-    host thread, engine (weights shared) and request stream per request; a round's requests start
-    together (a barrier) and each is timed from the round's start to its own logprobs. One warm-up
-    round first. Run only with --concurrent-ttft (CONCURRENT_TTFT_NOTE)."""
-    import threading
-
-    from chunkkv_amd.engine import HipEngine
-
-    streams = request_streams(n_streams, dev)
-    engines = [HipEngine(model, _Tok()) for _ in range(n_streams)]
-    times: list[float] = []
-    errors: list[BaseException] = []
-    for rnd in range(rounds + 1):
-        toks = [torch.randint(0, vocab, (N,), generator=torch.Generator().manual_seed(1000 + rnd * n_streams + j)).tolist()
-                for j in range(n_streams)]
-        start = threading.Barrier(n_streams + 1)
-        t0 = [0.0]
-        out = [0.0] * n_streams
-
-        def run(j):
-            try:
-                torch.cuda.set_device(dev)
-                with torch.cuda.stream(streams[j]):
-                    start.wait()
-                    res = engines[j].prefill(toks[j], placements_of[(rnd * n_streams + j) % len(placements_of)], cfg)
-                    engines[j].last_logprobs(res)
-                    out[j] = (time.perf_counter() - t0[0]) * 1e3
-                    del res
-            except BaseException as e:  # reported below, after every thread ended
-                errors.append(e)
-                start.abort()
-
-        threads = [threading.Thread(target=run, args=(j,)) for j in range(n_streams)]
-        for th in threads:
-            th.start()
-        torch.cuda.synchronize()
-        t0[0] = time.perf_counter()
-        try:
-            start.wait()
-        except threading.BrokenBarrierError:
-            pass
-        for th in threads:
-            th.join()
-        if errors:
-            raise errors[0]
-        if rnd:
-            times += out
-    del engines
-    torch.cuda.synchronize()
-    return times
 
 
 def traffic_probe(steps: int, warmup: int, dev) -> dict:
@@ -1419,8 +1355,7 @@ def _config_summary(line: dict) -> dict:
         out["roofline"] = {k: rf[k] for k in ("kernel", "achieved", "peak", "frac", "bytes_per_launch", "avg_launch_us")
                            if k in rf}
     for k in ("ratios", "store_gib", "ms_per_step_eager", "ms_per_step_uncorrelated", "uncorrelated_over_correlated",
-              "ttft_p50_ms", "ttft_p99_ms", "ttft_requests", "ttft_p50_ms_concurrent", "ttft_p99_ms_concurrent",
-              "ttft_requests_concurrent", "ttft_note", "ttft_concurrent_note"):
+              "ttft_p50_ms", "ttft_p99_ms", "ttft_requests", "ttft_note", "ttft_concurrent_note"):
         if k in line:
             out[k] = line[k]
     return out
@@ -1455,13 +1390,15 @@ def main() -> None:
                     help="skip the config-2, config-3 and config-5 sub-measurements of the default line")
     ap.add_argument("--replay-ttft-requests", type=int, default=20)
     ap.add_argument("--concurrent-ttft", action="store_true",
-                    help="config 5: also time 4 concurrent HipEngine prefills (one host thread each; off by default)")
+                    help="switched off: concurrent HipEngine prefills stalled (ends with the reason)")
     ap.add_argument("--workload", default="request",
                     choices=["request", "gather", "deviation", "replay", "traffic", "dropped", "attention", "extract",
                              "decode", "layer1_32k"],
                     help="request: the 8k Qwen2.5-7B blend-prefill KV repair (default); gather / deviation / replay: "
                          "the re-RoPE+gather, deviation+top-k+scatter and 4x32k replay microbenchmarks")
     args = ap.parse_args()
+    if args.concurrent_ttft:
+        ap.error("--concurrent-ttft: " + CONCURRENT_TTFT_NOTE)
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) != 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (run with --gpus 1)", file=sys.stderr)
         sys.exit(2)
@@ -1473,8 +1410,7 @@ def main() -> None:
               "traffic": traffic_probe, "dropped": bench_dropped, "attention": bench_attention,
               "extract": bench_extract, "decode": bench_decode, "layer1_32k": bench_layer1_32k}[args.workload]
         if args.workload == "replay":
-            print(json.dumps(bench_replay(args.steps, args.warmup, dev, ttft_requests=args.replay_ttft_requests,
-                                          concurrent_ttft=args.concurrent_ttft)),
+            print(json.dumps(bench_replay(args.steps, args.warmup, dev, ttft_requests=args.replay_ttft_requests)),
                   flush=True)
         else:
             print(json.dumps(fn(args.steps, args.warmup, dev)), flush=True)
@@ -1495,8 +1431,7 @@ def main() -> None:
         log(f"[bench] config 3 {configs['config3_deviation_topk_scatter']}")
         # before the 8k TTFT runs, like the sub-measurements above; it builds its own model
         configs["config5_replay"] = _config_summary(
-            bench_replay(min(args.steps, 20), args.warmup, dev, ttft_requests=args.replay_ttft_requests,
-                         concurrent_ttft=args.concurrent_ttft))
+            bench_replay(min(args.steps, 20), args.warmup, dev, ttft_requests=args.replay_ttft_requests))
         log(f"[bench] config 5 {configs['config5_replay']}")
     ttft = bench_ttft(args.ttft_requests, dev) if args.ttft_requests > 0 else None
     model = ttft.pop("model") if ttft is not None else None
