@@ -20,7 +20,8 @@
 // conflict-free; V^T comes out of row-major V through transposing LDS reads. Scores and the output accumulate in
 // fp32; P is rounded to bf16 for the second product (as fused SDPA kernels do). Launches with too
 // few 128-query workgroups to fill the chip (decode, short prompts, small blends) run
-// attention_wave.hpp's kernel instead. Built with the MFMA VGPR form (no accumulator-register
+// attention_wave.hpp's kernel instead, or, over a long cache, this one in splits of the cache whose
+// partial rows attn_combine_kernel merges (attention_plan.hpp). Built with the MFMA VGPR form (no accumulator-register
 // copies around the online-softmax rescale).
 // Bound: issue and power together. The matrix cores run half of the cycles and the vector
 // instructions most of the rest, so every vector instruction that is not softmax costs time: tile
@@ -120,12 +121,13 @@ __device__ __forceinline__ bool attn_work_item(int nqb, int group, int xpk_log, 
   return j < items;
 }
 
-template <int D>
+// SPLIT: split z of the cache's tiles per workgroup, unnormalised rows with their max and sum to ws.
+template <int D, bool SPLIT>
 __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
     int nqb, int map_group, int xpk_log, int items, uint32_t inv_group, uint32_t inv_nqb,
     const int64_t* __restrict__ pos, int n, int N, const char* __restrict__ kc, const char* __restrict__ vc,
     int64_t kv_hs_b, const char* __restrict__ q, int64_t q_hs_b, int64_t q_ts_b, int Hq, int group, float scale_log2,
-    char* __restrict__ out, int32_t* __restrict__ err) {
+    char* __restrict__ out, int32_t* __restrict__ err, float* __restrict__ ws, int split_tiles) {
   constexpr int DS = D / 32;          // k-steps of S^T = K Q^T
   constexpr int DT = D / 16;          // 16-row tiles of O^T
   constexpr int CPR = D / 8;          // 16-byte chunks per cache row
@@ -177,7 +179,9 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
 #pragma unroll
   for (int w = 1; w < kAttnWaves; ++w) bmax = max(bmax, blk_max_s[w]);
   bmax = __builtin_amdgcn_readfirstlane(bmax);
-  const int n_tiles = bmax < 0 ? 0 : bmax / kAttnBN + 1;
+  int n_tiles = bmax < 0 ? 0 : bmax / kAttnBN + 1;
+  const int tile_begin = SPLIT ? z * split_tiles : 0;
+  if (SPLIT) n_tiles = min(n_tiles, tile_begin + split_tiles);
 
   // Q fragments (B operand of S^T): query q0 + 16 qg + lm, head-dim 32 s + 8 g .. + 8.
   bf16x8 qf[kAttnQG][DS];
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
   int k_rd[DS];
 #pragma unroll
   for (int ds = 0; ds < DS; ++ds) k_rd[ds] = lm * ROWB + (((4 * ds + g) ^ swz_k<CPR>(lm)) * 16);
-  if (n_tiles > 0) issue(0, k_lds0, v_lds0);
+  if (tile_begin < n_tiles) issue(tile_begin * kAttnBN, k_lds0, v_lds0);
 
   // One tile; the loop below alternates the buffers (each call names its buffers directly, so
   // the compiler sees that the loads in flight never alias the buffer being read).
@@ -355,7 +359,7 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
         }
       }
   };
-  for (int tile = 0; tile < n_tiles; tile += 2) {
+  for (int tile = tile_begin; tile < n_tiles; tile += 2) {
     body(tile, k_lds0, v_lds0, k_lds1, v_lds1);
     if (tile + 1 < n_tiles) body(tile + 1, k_lds1, v_lds1, k_lds0, v_lds0);
   }
@@ -366,6 +370,16 @@ __global__ __launch_bounds__(kAttnWaves * 64) void attn_active_kernel(
     const float l = l_acc[qg][0];
     const int m = q0 + qg * 16 + lm;
     if (m >= n) continue;
+    if (SPLIT) {
+      float* prow = ws + (((int64_t)z * Hq + hq) * n + m) * (D + 4);  // 16-byte aligned rows
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) *(f32x4*)(prow + dt * 16 + 4 * g) = o[qg][dt];
+      if (g == 0) {
+        prow[D] = m_run[qg];
+        prow[D + 1] = l;
+      }
+      continue;
+    }
     const float inv = 1.f / l;
     char* orow = out + ((int64_t)m * Hq + hq) * (D * 2);
 #pragma unroll
@@ -386,7 +400,7 @@ extern "C" int64_t ckv_attention_workspace_bytes(int32_t n_queries, int32_t n_to
                                                  int32_t head_dim, int32_t* splits_out, int32_t* split_tiles_out) {
   using namespace ckv;
   const bool some = n_queries > 0 && n_tokens > 0 && n_q_heads > 0 && head_dim > 0;
-  const int64_t splits = some ? most_splits(n_queries, n_tokens, n_q_heads, head_dim) : 1;
+  const int64_t splits = some ? attn_most_splits(n_queries, n_tokens, n_q_heads, head_dim) : 1;
   const int tiles = n_tokens > 0 ? (n_tokens + kAttnBN - 1) / kAttnBN : 0;
   if (splits_out != nullptr) *splits_out = (int32_t)splits;
   if (split_tiles_out != nullptr) *split_tiles_out = splits > 1 ? (int32_t)((tiles + splits - 1) / splits) : 0;
@@ -417,34 +431,33 @@ extern "C" int32_t ckv_attention_active(void* out, const void* q, int64_t q_head
   const AttnPlan plan = attn_plan(n_queries, n_tokens, n_q_heads, n_kv_heads, head_dim,
                                   workspace != nullptr && (uintptr_t)workspace % 16 == 0 ? workspace_bytes : 0);
   const AttnMap& map = plan.map;
-  if (!plan.wave) {
+  float* ws = plan.splits > 1 ? (float*)workspace : nullptr;
+  if (plan.wave) {
+    const uint32_t inv_gqa = inverse_of((int64_t)n_queries * group, group);
+    auto launch = [&](auto kernel, int waves) {
+      hipLaunchKernelGGL(kernel, dim3(map.blocks), dim3(waves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
+                         map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
+                         (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
+                         n_q_heads, group, inv_gqa, scale_log2, plan.split_chunks, (char*)out, ws, err);
+    };
+#define CKV_WAVE(HD, QG, W, GR) \
+  else if (head_dim == HD && plan.qg == QG && plan.waves == W && plan.grouped == GR) \
+    launch(attn_wave_kernel<HD, QG, W, GR>, W);
+    if (false) {
+    }
+    CKV_WAVE_FORMS(CKV_WAVE)
+    else return CKV_ERR_INVALID_ARGUMENT;  // a plan outside the list
+#undef CKV_WAVE
+  } else {
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(map.blocks), dim3(kAttnWaves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
                          map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
                          (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
-                         n_q_heads, group, scale_log2, (char*)out, err);
+                         n_q_heads, group, scale_log2, (char*)out, err, ws, plan.split_chunks / (kAttnBN / kWaveChunk));
     };
-    if (head_dim == 128) launch(attn_active_kernel<128>);
-    else launch(attn_active_kernel<64>);
-    CKV_RETURN_IF_LAUNCH_FAILED();
-    return CKV_OK;
+    if (head_dim == 128) ws != nullptr ? launch(attn_active_kernel<128, true>) : launch(attn_active_kernel<128, false>);
+    else ws != nullptr ? launch(attn_active_kernel<64, true>) : launch(attn_active_kernel<64, false>);
   }
-  float* ws = plan.splits > 1 ? (float*)workspace : nullptr;
-  const uint32_t inv_gqa = inverse_of((int64_t)n_queries * group, group);
-  auto launch = [&](auto kernel, int waves) {
-    hipLaunchKernelGGL(kernel, dim3(map.blocks), dim3(waves * 64), 0, st, map.nqb, map.group, map.xpk_log, map.items,
-                       map.inv_group, map.inv_nqb, positions, n_queries, n_tokens, (const char*)k_cache,
-                       (const char*)v_cache, kv_head_stride * 2, (const char*)q, q_head_stride * 2, q_token_stride * 2,
-                       n_q_heads, group, inv_gqa, scale_log2, plan.split_chunks, (char*)out, ws, err);
-  };
-#define CKV_WAVE(HD, QG, W, GR) \
-  else if (head_dim == HD && plan.qg == QG && plan.waves == W && plan.grouped == GR) \
-    launch(attn_wave_kernel<HD, QG, W, GR>, W);
-  if (false) {
-  }
-  CKV_WAVE_FORMS(CKV_WAVE)
-  else return CKV_ERR_INVALID_ARGUMENT;  // a plan outside the list
-#undef CKV_WAVE
   CKV_RETURN_IF_LAUNCH_FAILED();
   if (ws != nullptr) {
     const dim3 grid((unsigned)n_queries, (unsigned)n_q_heads);

@@ -59,6 +59,7 @@ int main() {
               if (p.splits > 1)
                 ok = ok && p.splits * row_b <= ws && p.splits * row_b <= need && (int64_t)p.splits * p.split_chunks >= chunks &&
                      (int64_t)(p.splits - 1) * p.split_chunks < chunks;
+              ok = ok && (p.wave || p.split_chunks % (kAttnBN / kWaveChunk) == 0);  // whole tiles
               ok = ok && (p.map.blocks > 3000 || items_once(p, Hq, Hkv));
               ++checked;
               if (!ok && bad++ < 10)
@@ -66,6 +67,12 @@ int main() {
                             Hq, Hkv, D, n, N, (long long)ws, p.wave, p.qg, p.waves, p.grouped, p.splits, p.split_chunks, (long long)chunks);
             }
           }
+  // the large kernel in splits, at the shapes that the GPU test of it runs
+  const int split[][5] = {{28, 4, 128, 5120, 130}, {7, 7, 128, 9001, 700}, {32, 8, 64, 9000, 251}, {12, 3, 64, 8300, 333}};
+  for (const auto& t : split) {
+    const AttnPlan p = attn_plan(t[4], t[3], t[0], t[1], t[2], (int64_t)1 << 50);
+    if (p.wave || p.splits < 2) ++bad, std::printf("not split: %d queries over %d\n", t[4], t[3]);
+  }
   std::printf("%ld %ld\n", checked, bad);
   return 0;
 }

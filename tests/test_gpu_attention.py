@@ -166,3 +166,24 @@ def test_attention_more_kv_heads_than_a_grouped_launch_fills(Hq, Hkv, D, N, n):
     out, e = _run(q, K, V, pos)
     assert e == 0
     np.testing.assert_allclose(out[0].float().cpu().numpy(), O.attention_active(q, K, V, pos), atol=ATOL, rtol=0)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,N,n", [
+    (28, 4, 128, 5120, 130),  # ten splits of eight tiles, the second query block two rows
+    (7, 7, 128, 9001, 700),   # no grouping, the last split and the last tile ragged
+    (32, 8, 64, 9000, 251),
+    (12, 3, 64, 8300, 333),   # KV heads that do not divide the 8 XCDs
+])
+def test_attention_large_kernel_in_splits(Hq, Hkv, D, N, n):
+    """128-query workgroups over splits of a long cache: against the oracle and unsplit, with a query at
+    position 0 (it sees one row of the first split and none of the others) and the rows past every
+    position uninitialised (NaN). Tolerance as at the top of this file."""
+    q, K, V, pos = _case(N + n, Hq, Hkv, D, N, n)
+    seen = N - 3
+    pos = np.minimum(pos, seen - 1)
+    K[:, seen:], V[:, seen:] = 0x7FC0, 0x7FC0
+    args = [O.from_numpy(a, DEV)[None] for a in (q, K, V)] + [torch.from_numpy(pos).to(DEV)]
+    sub = np.unique(np.r_[0, 1, np.linspace(0, n - 1, min(n, 120)).astype(int)])
+    want = O.attention_active(q[:, sub], K[:, :seen], V[:, :seen], pos[sub])
+    for out in (ops.attention_active(*args), ops.attention_active(*args, split=False)):
+        np.testing.assert_allclose(out[0].float().cpu().numpy()[sub], want, atol=ATOL, rtol=0)
