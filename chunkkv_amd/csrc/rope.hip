@@ -14,8 +14,8 @@
 // from theta, passed by value in the kernel arguments) and each token's position, evaluated in
 // fp64 with the short reduction + series of cos_sin.hpp. A k/v-only launch (the cache repair)
 // runs one wavefront per token, each lane evaluating one frequency once and the lanes sharing
-// them through ds_bpermute, and so does a launch with q (head_dim 256: each evaluation shared over 4
-// heads). A caller-kept
+// them through ds_bpermute, and so does a launch with q (head_dim 256, and a few tokens of many heads:
+// each evaluation shared over 4 heads). A caller-kept
 // per-position table (ckv_rope_table) is also accepted. All accesses are 16 bytes. The ~20 elementwise torch
 // launches of the reference's RoPE (fp32 temporaries, cat, cast) and the separate scatter of k/v
 // into the cache become one pass over the projection output.
@@ -292,6 +292,9 @@ __global__ __launch_bounds__(kRopeKvThreads) void rope_kv_kernel(
   }
 }
 
+constexpr int kRopeTokenNB = 5;      // items a lane of rope_token_kernel in one batch of loads, at most
+constexpr int kRopeTokenMany = 640;  // launches of more tokens take it with any number of items
+
 // Without a table, with q, head_dim <= 128: one wavefront per token, as rope_kv_kernel. Item i of a
 // token is the 16-byte column pair (col, col + D/2) of head row i / TPR: q heads, then k heads
 // (rotated), then v heads (copied); lane l takes items l, l + 64, ... and its first NB items' loads
@@ -374,7 +377,7 @@ __global__ __launch_bounds__(kRopeKvThreads) void rope_token_kernel(
   }
 }
 
-// Without a table, with q, head_dim 256: one thread per
+// Without a table, with q, head_dim 256 or a small launch of many heads: one thread per
 // (token, 16-byte column, group of kRopeFreeHG heads), grid-stride, evaluating its VEC
 // frequencies itself (kRopeFreeHG-fold sharing), v copied in 16-byte chunks. The thread's loads go
 // out in the order their values are needed (position, row, inverse frequencies, data) and it
@@ -587,6 +590,11 @@ static void launch_rope(int n, hipStream_t st, char* qo, int64_t qo_hs, int64_t 
     return;
   }
   if constexpr (D <= 2 * kWave) {
+    // Tokens of more items than one batch of loads cost this form a second dependent round trip, which
+    // small launches are made of: those keep the form that spreads a token over threads (64 + 8 + 8
+    // heads of 128, this form first: 64 tokens 6.6 and 5.2 us, 500 8.1 and 7.8, 1000 9.4 and 11.1, 8256
+    // 60.7 and 65.9; 28 + 4 + 4 in fp32 4.2 and 3.9, 5.6 and 5.1, 6.4 and 7.3, 48.7 and 51.4; nine to
+    // twelve items a lane in one batch: 6.6 for the 64 tokens).
     const int items = (Hq + Hkv + (vo != nullptr ? Hkv : 0)) * (D / 2 / Elem<DTYPE>::kVec);
     auto go = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(kRopeKvThreads), 0, st, n, Hq, Hkv, items, pos, qi, ki, vi, qi_hs,
@@ -599,18 +607,20 @@ static void launch_rope(int n, hipStream_t st, char* qo, int64_t qo_hs, int64_t 
       else if (rows == pos) go(rope_token_kernel<DTYPE, D, kRowPos, NB>);
       else go(rope_token_kernel<DTYPE, D, kRowIndexed, NB>);
     };
-    if (items <= 2 * kWave) batch(std::integral_constant<int, 2>{});
-    else if (items <= 3 * kWave) batch(std::integral_constant<int, 3>{});
-    else batch(std::integral_constant<int, 5>{});
-  } else {
-    using E = Elem<DTYPE>;
-    const int64_t per_tok = (int64_t)(Hq + Hkv + kRopeFreeHG - 1) / kRopeFreeHG * (D / 2 / E::kVec) +
-                            (vo != nullptr ? Hkv * (D * E::kBytes / 16) : 0);
-    const int64_t blocks = std::min<int64_t>((n * per_tok + kRopeThreads - 1) / kRopeThreads, 1 << 20);
-    hipLaunchKernelGGL((rope_free_kernel<DTYPE, D>), dim3((unsigned)blocks), dim3(kRopeThreads), 0, st, qo, qo_hs, qo_ts,
-                       ko, ko_hs, ko_ts, vo, vo_hs, vo_ts, rows, n_out, qi, qi_hs, qi_ts, ki, ki_hs, ki_ts, vi, vi_hs,
-                       vi_ts, pos, inv, n, Hq, Hkv, err);
+    if (items <= kRopeTokenNB * kWave || n > kRopeTokenMany) {
+      if (items <= 2 * kWave) batch(std::integral_constant<int, 2>{});
+      else if (items <= 3 * kWave) batch(std::integral_constant<int, 3>{});
+      else batch(std::integral_constant<int, kRopeTokenNB>{});
+      return;
+    }
   }
+  using E = Elem<DTYPE>;
+  const int64_t per_tok = (int64_t)(Hq + Hkv + kRopeFreeHG - 1) / kRopeFreeHG * (D / 2 / E::kVec) +
+                          (vo != nullptr ? Hkv * (D * E::kBytes / 16) : 0);
+  const int64_t blocks = std::min<int64_t>((n * per_tok + kRopeThreads - 1) / kRopeThreads, 1 << 20);
+  hipLaunchKernelGGL((rope_free_kernel<DTYPE, D>), dim3((unsigned)blocks), dim3(kRopeThreads), 0, st, qo, qo_hs, qo_ts,
+                     ko, ko_hs, ko_ts, vo, vo_hs, vo_ts, rows, n_out, qi, qi_hs, qi_ts, ki, ki_hs, ki_ts, vi, vi_hs,
+                     vi_ts, pos, inv, n, Hq, Hkv, err);
 }
 
 typedef void (*RopeLaunch)(int, hipStream_t, char*, int64_t, int64_t, char*, int64_t, int64_t, char*, int64_t,

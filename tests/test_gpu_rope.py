@@ -229,7 +229,11 @@ def test_rope_kv_every_row_mode_and_shape(shape, row_mode, n):
     (False, 64, 20, 2, 7),   # 192: exactly three
     (True, 128, 28, 4, 129), # 288: the last of five part full
     (True, 128, 32, 4, 5),   # 320: exactly five
-    (False, 128, 33, 8, 9),  # 784: batches after the first
+    (False, 128, 33, 8, 9),  # 784: a token spread over threads
+    (False, 128, 33, 8, 640),  # the last such launch
+    (False, 128, 33, 8, 641),  # batches after the first
+    (True, 128, 64, 8, 700),   # 640: exactly two batches
+    (True, 128, 33, 4, 11),    # 328: one item past a batch
 ])
 def test_rope_qkv_items_per_token(bf16, D, Hq, Hkv, n):
     """Every batch size of the one-wavefront-per-token kernel at its edges, in its three row modes
