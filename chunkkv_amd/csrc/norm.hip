@@ -90,15 +90,15 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_kernel(char* h_out, 
   }
 }
 
-// The gated product: a thread takes one 16-byte column of kGateRows rows, all its loads in flight
-// together. Bound: HBM. gate and up are read once (non-temporal loads); the product is stored with
-// device scope, written through the L2 so that no dirty lines wait for the end of the launch, and
-// stays where the down projection that reads it next finds it. 2976 rows of 18944 (338 MB): 60.0 us
-// with one row and regular accesses, 58.5 with non-temporal loads, 55.4 with two rows and these
-// stores (6.1 TB/s), 59-67 with four or eight rows; followed by the product that reads it 600.0
-// -> 594.9 us (non-temporal stores 602.1).
-constexpr int kGateRows = 2;
-
+// The gated product: a thread takes one 16-byte column of a row. Bound: HBM, at few rows the launch.
+// gate and up are read once (non-temporal loads); the product is stored with device scope, written
+// through the L2 so that no dirty lines wait for the end of the launch, and stays where the down
+// projection that reads it next finds it. With regular accesses, with these, and with these and two
+// rows a thread (us, graph replays): 2976 rows of 18944 (338 MB) 59.9, 50.9 (6.6 TB/s), 52.7; 8256
+// rows 172.8, 161.4, 168.1; 64 rows of 14336 2.8, 2.6, 3.4; 251 rows of 4864 3.0, 2.9, 3.3. Slower only
+// where a replay finds its operands in the last-level cache (8256 rows of 4864 35.5, 37.9, 36.3; the
+// steps of a layer around it 72.3 and, with two rows, 72.7). Followed by the product that reads it
+// 599 -> 594 us at 2976 rows of 18944 (non-temporal stores 602).
 template <int DTYPE>
 __global__ __launch_bounds__(kGateThreads) void silu_mul_kernel(char* __restrict__ out, int64_t out_rs_b,
                                                                 const char* __restrict__ gate, int64_t gate_rs_b,
@@ -108,30 +108,19 @@ __global__ __launch_bounds__(kGateThreads) void silu_mul_kernel(char* __restrict
   const int v = blockIdx.x * kGateThreads + threadIdx.x;
   if (v >= vecs_per_row) return;
   const int64_t cb = (int64_t)v * 16;
-  for (int64_t r0 = (int64_t)blockIdx.y * kGateRows; r0 < n_rows; r0 += (int64_t)gridDim.y * kGateRows) {
-    vec16 a[kGateRows], b[kGateRows];
+  for (int64_t row = blockIdx.y; row < n_rows; row += gridDim.y) {
+    float g[E::kVec], u[E::kVec], o[E::kVec];
+    E::unpack(ld16_stream(gate + row * gate_rs_b + cb), g);
+    E::unpack(ld16_stream(up + row * up_rs_b + cb), u);
 #pragma unroll
-    for (int j = 0; j < kGateRows; ++j) {  // a row past the end: the last one again, not stored
-      const int64_t row = r0 + j < n_rows ? r0 + j : n_rows - 1;
-      a[j] = ld16_stream(gate + row * gate_rs_b + cb);
-      b[j] = ld16_stream(up + row * up_rs_b + cb);
+    for (int e = 0; e < E::kVec; ++e) {
+      // exp(-g) = 2^(-g log2 e) and 1/den on the hardware's exp2 and reciprocal (about 1 ulp
+      // each in fp32), not the library's exp and IEEE division: a third of the VALU work,
+      // which otherwise bounds the kernel at the 8k request's width
+      const float den = 1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g[e]);
+      o[e] = E::round_trip(g[e] * __builtin_amdgcn_rcpf(den)) * u[e];
     }
-#pragma unroll
-    for (int j = 0; j < kGateRows; ++j) {
-      if (r0 + j >= n_rows) break;
-      float g[E::kVec], u[E::kVec], o[E::kVec];
-      E::unpack(a[j], g);
-      E::unpack(b[j], u);
-#pragma unroll
-      for (int e = 0; e < E::kVec; ++e) {
-        // exp(-g) = 2^(-g log2 e) and 1/den on the hardware's exp2 and reciprocal (about 1 ulp
-        // each in fp32), not the library's exp and IEEE division: a third of the VALU work,
-        // which otherwise bounds the kernel at the 8k request's width
-        const float den = 1.0f + __builtin_amdgcn_exp2f(-1.44269504088896341f * g[e]);
-        o[e] = E::round_trip(g[e] * __builtin_amdgcn_rcpf(den)) * u[e];
-      }
-      st16_agent(out + (r0 + j) * out_rs_b + cb, E::pack(o));
-    }
+    st16_agent(out + row * out_rs_b + cb, E::pack(o));
   }
 }
 
@@ -169,8 +158,7 @@ int launch_silu_mul(void* out, int64_t out_rs, const void* gate, int64_t gate_rs
   if (out_rs % E::kVec != 0 || gate_rs % E::kVec != 0 || up_rs % E::kVec != 0) return CKV_ERR_INVALID_ARGUMENT;
   const int vpr = width / E::kVec;
   const unsigned col_blocks = (unsigned)((vpr + kGateThreads - 1) / kGateThreads);
-  const int64_t row_groups = (n_rows + kGateRows - 1) / kGateRows;
-  const unsigned row_blocks = (unsigned)(row_groups < kGateMaxRowBlocks ? row_groups : kGateMaxRowBlocks);
+  const unsigned row_blocks = (unsigned)(n_rows < kGateMaxRowBlocks ? n_rows : kGateMaxRowBlocks);
   hipLaunchKernelGGL(silu_mul_kernel<DTYPE>, dim3(col_blocks, row_blocks), dim3(kGateThreads), 0, stream,
                      (char*)out, out_rs * E::kBytes, (const char*)gate, gate_rs * E::kBytes, (const char*)up,
                      up_rs * E::kBytes, n_rows, vpr);
