@@ -345,6 +345,36 @@ def test_rerope_gather_segment_count_limits(n_segs):
 
 
 
+@pytest.mark.parametrize("most", [16, 64, 128])
+def test_rerope_gather_many_ragged_segments(most):
+    """64 or more segments of very different lengths, the longest a whole even number of tiles: the
+    launch that pads its tile count. Every row lands, bit for bit, with and without a skip map."""
+    rng = np.random.default_rng(most)
+    H, D, n_segs = 2, 128, 70
+    lens = np.where(np.arange(n_segs) % 7 == 3, most, rng.integers(1, 17, n_segs))
+    at = np.concatenate([[0], np.cumsum(lens)])
+    N = int(at[-1])
+    k, v = (O.f32_to_bf16_bits(rng.standard_normal((H, N, D)).astype(np.float32)) for _ in range(2))
+    kt, vt = O.from_numpy(k, DEV), O.from_numpy(v, DEV)
+    segs = np.stack([at[:-1], lens, np.zeros(n_segs), at[:-1], np.full(n_segs, N), rng.integers(-900, 900, n_segs)], 1).astype(np.int32)
+    tab = torch.tensor([kt.data_ptr(), vt.data_ptr()], dtype=torch.int64, device=DEV)
+    skip = np.where(rng.random(N) < 0.2, 1, -1).astype(np.int32)
+    want = np.zeros((2, 1, H, N, D), dtype=np.uint16)
+    assert O.rerope_gather(want[0], want[1], [[k]], [[v]], segs, THETA) == 0
+    for skipped in (None, skip):
+        K = torch.zeros((1, 1, H, N, D), dtype=torch.bfloat16, device=DEV)
+        V = torch.zeros_like(K)
+        err = torch.zeros(1, dtype=torch.int32, device=DEV)
+        ops.rerope_gather(K, V, tab, torch.from_numpy(segs.reshape(-1)).to(DEV), n_segs, int(lens.max()), THETA, err,
+                          skip=None if skipped is None else torch.from_numpy(skipped).to(DEV))
+        assert int(err.item()) == 0
+        rows = slice(None) if skipped is None else skipped < 0
+        np.testing.assert_array_equal(O.to_numpy(K)[0, 0][:, rows], want[0, 0][:, rows])
+        np.testing.assert_array_equal(O.to_numpy(V)[0, 0][:, rows], want[1, 0][:, rows])
+        if skipped is not None:
+            assert not O.to_numpy(K)[0, 0][:, skipped >= 0].any()
+
+
 def test_rerope_gather_flags_bad_segment_without_writing():
     H, D, N = 2, 64, 32
     src = torch.randn((1, H, 8, D), device=DEV)
