@@ -4,8 +4,9 @@ hand-written gfx950 kernels.
 Public surface = src/chunkkv/engine/torch_engine.py:18-207: constructor ``(model, tokenizer)``,
 ``load(repo, dtype)``, ``prefill(tokens, placements, config, logits_from) -> PrefillResult``,
 ``generate``, ``last_logprobs``, ``sync``, ``clear_cache``, ``shift_keys``, ``tokenizer``.
-The model's GEMMs, RMSNorm and MLP stay on PyTorch-ROCm (chunkkv_amd.model). The KV repair,
-the fresh-token RoPE and the attention run on the HIP kernels:
+The model's large GEMMs stay on PyTorch-ROCm (chunkkv_amd.model). The KV repair, the fresh-token
+RoPE, the attention, the steps between the GEMMs and the projections of short requests run on the HIP
+kernels:
 
   reference (torch_engine.py)                        here
   _qkv + _rope/_rotate (:61-66, :53-54, :46-51)      one q|k|v GEMM (stacked weights), then
@@ -77,6 +78,7 @@ import numpy as np
 import torch
 import torch.nn.functional as F
 from torch.nn.attention import SDPBackend, sdpa_kernel
+from torch.nn.modules.module import _has_any_global_hook
 
 from chunkkv_amd import _native, ops
 from chunkkv_amd.model import DecoderPieces
@@ -133,17 +135,18 @@ def _stack_params(mods: list, name: str) -> torch.Tensor | None:
     return stacked
 
 
-_LINEAR_FORWARD = torch.nn.Linear.forward
+_LINEAR, _LINEAR_FORWARD = torch.nn.Linear, torch.nn.Linear.forward
 
 
 def _apply_linear(m, x: torch.Tensor) -> torch.Tensor:
     """m(x); for an nn.Linear that nothing wraps, hooks, compiles or patches, its product by ops.linear."""
-    p = m._parameters
-    if (type(m) is torch.nn.Linear and torch.nn.Linear.forward is _LINEAR_FORWARD and "forward" not in m.__dict__
-            and m._compiled_call_impl is None and "weight" in p and "bias" in p
-            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
-            and not torch.nn.modules.module._has_any_global_hook()):
-        return ops.linear(x, p["weight"], p["bias"])
+    if type(m) is _LINEAR and _LINEAR.forward is _LINEAR_FORWARD:
+        d = m.__dict__
+        p = d["_parameters"]
+        if "weight" in p and "bias" in p and not (
+                d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or "forward" in d or d.get("_compiled_call_impl") is not None or _has_any_global_hook()):
+            return ops.linear(x, p["weight"], p["bias"])
     return m(x)
 
 
