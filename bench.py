@@ -1133,7 +1133,7 @@ def bench_extract(steps: int, warmup: int, dev) -> dict:
         "store-put extraction, HBM GB/s", nb / (ms * 1e-3) / 1e9, ms, steps, warmup,
         {"workload": "24 reusable segments x 320 tokens of the 8256-token request, 28 layers, 4 KV heads, "
                      "head_dim 128, bf16, one launch (value: the whole PrefillResult.chunks call, incl. the 24 "
-                     "buffer allocations and the descriptor copy)"},
+                     "buffer allocations)"},
         _rooffor("extract_kernel", nb, ms_k))
     line["reference_per_layer_copies_ms"] = round(ms_ref, 4)
     return line

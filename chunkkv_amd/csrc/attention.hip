@@ -27,8 +27,10 @@
 // instructions most of the rest, so every vector instruction that is not softmax costs time: tile
 // addresses are a kept offset on a uniform base (62 -> 8 instructions a tile), wavefront extremes
 // are scalar (branches, not selects), the four lanes of a query agree on its max only where a lane
-// asks to raise it. Measured (us, 28 heads of 128): 2976 rows over 8256 216 -> 196 (1010 TFLOP/s),
-// 8256 causal rows 480 -> 449 (1089), 2000 51.2 -> 47.4; 14 heads of 64, 8256 causal rows 162 -> 144.
+// asks to raise it. Measured (us, 28 heads of 128): 2976 rows over 8256, 216 -> 196 with the
+// rows spread evenly (199 GFLOP: 1010 TFLOP/s) and 234 -> 216 as a blend keeps them, most in the chunks
+// that moved (215 GFLOP: 996; 203-226 on other cards); 8256 causal rows 480 -> 449 (1089), 2000 51.2 ->
+// 47.4; 14 heads of 64, 8256 causal rows 162 -> 144.
 // A square bf16 product of 8192 reaches 1300-1400 on this card; inputs of zeros (no toggling) 10 %
 // more than these. Not faster: tiles one ahead so that the matrix cores work beside the exponentials
 // (209-214 / 478 before this form, with spills), V operands read ahead of their products (the same),

@@ -1,5 +1,5 @@
 // The attention of a launch too small for 128-query workgroups to fill the chip: decode, short
-// prompts, the few rows of a small blend. Included by attention.hip, whose layouts it shares.
+// prompts, the few rows of a small blend (attention_plan.hpp says which). Included by attention.hip, whose layouts it shares.
 //
 // Bound: latency. A 128-query workgroup that walks the cache one 64-row tile at a time is a chain
 // of dependent steps (load, barrier, product, softmax, product) as long as the cache, and a launch
@@ -53,14 +53,13 @@ __global__ __launch_bounds__(W * 64) void attn_wave_kernel(
   const int hk = GROUPED ? hq : div_by(hq, group, inv_gqa);
   if (GROUPED) hq *= group;  // the KV head's first query head
   const int n_rows = GROUPED ? n * group : n;
-  int row_m[QG], row_h[QG];  // token and query head of this lane's rows (row_m == n: no query)
+  int row_m[QG];  // token of this lane's rows (n: no query)
   int64_t p64[QG];
 #pragma unroll
   for (int qg = 0; qg < QG; ++qg) {
     const int r = qb * ROWS + qg * 16 + lm;
     const int t = GROUPED ? div_by(r, group, inv_gqa) : r;
     row_m[qg] = r < n_rows ? t : n;
-    row_h[qg] = GROUPED ? hq + r - t * group : hq;
     p64[qg] = pos[min(row_m[qg], n - 1)];
   }
 

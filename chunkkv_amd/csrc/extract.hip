@@ -26,8 +26,9 @@ constexpr int kExtractTile = 8;
 // Up to 64 segments by value (1 KB of kernel arguments): a table in device memory costs a pinned
 // block and a copy in front of the launch, and each workgroup a dependent load of its span. The 8k
 // request's whole call (24 segments x 320 tokens x 28 layers, calls back to back, both builds
-// alternating): 156.4-156.6 -> 149.2-149.4 us on one box, 161.7 -> 155.8-156.7 us on another. Longer
-// lists keep the table: the arguments of one launch are bounded (4 KB).
+// alternating, one line a card): 156.4-156.6 -> 149.2-149.4 us, 154.1 -> 146.3, 161.7 -> 155.8-156.7,
+// 159.0 -> 154.8 (the last two within a few per cent of noise). 64 is a chosen size, not a measured
+// edge: arguments hold about 250 segments (4 KB), and longer lists were not measured in this form.
 constexpr int kExtractArgs = 64;
 struct ExtractSpans {
   uint64_t dst[kExtractArgs];

@@ -204,10 +204,16 @@ static LinPlan linear_plan(int64_t M, int64_t N, int64_t K, int64_t workspace_by
   return p;
 }
 
-// Where this beats the library: not for one row (decode replays a graph, so the host does not count,
-// and the library's one-row kernels are faster: 1152 x 896 4.2 us against 6.2), and up to 5 GFLOP,
-// about where the library's kernels take as long as its host call (1103 rows of 9728 x 896, 19
-// GFLOP: 24.6 us against 32).
+// Where calls issued one after the other gain from this: not for one row (decode replays a graph, so
+// the host does not count, and the library's one-row kernels are faster: 1152 x 896 4.2 us against
+// 6.2), and up to 5 GFLOP, about where the library's kernels take as long as its host call (1103 rows
+// of 9728 x 896, 19 GFLOP: 24.6 us against 32). It is the host time that this bounds, 4 us a call
+// against 20; the kernels alone (us, this first, graph replays over weights as a model reads them,
+// without the committed GEMM table): 7B shapes, 2-32 rows, q|k|v 10.4-11.4 and 12.5-13.3, o 9.3-10.2 and
+// 12.0, down 27-30.5 and 46-110, gate|up (to 16 rows) 54-56 and 54-55; 0.5B shapes, 2-24 rows, q|k|v
+// and o 6.2-6.5 and 5.6, gate|up 7.0 and 8.7, down 7.2-7.9 and 12.8; 1103 rows of q|k|v and o 10.3 and
+// 9.0, 251 of gate|up 17.8 and 15.1. By kernel time alone the lines would lie elsewhere (64 rows of
+// 3584 x 18944, left to the library, take it 85.8 us and this 28.9).
 constexpr int64_t kLinMaxWork = 2500000000;  // n_rows * n_out * n_in
 
 }  // namespace ckv

@@ -546,8 +546,9 @@ int32_t ckv_attention_active(void* out, const void* q, int64_t q_head_stride, in
 /*
  * Bytes of workspace ckv_attention_active uses to split a launch of this shape (0: it never
  * splits this shape): partial rows of the most splits that it may take, over all group sizes. With
- * less than that, or none, it takes fewer. That split count and the cache tiles (64 rows) of one
- * split go to *splits and *split_tiles when those are not NULL. Host-only, no device work. No
+ * less than that, or none, it takes fewer. That split count goes to *splits and the cache tiles (64
+ * rows, rounded up) that each of so many splits would have to *split_tiles when those are not NULL; a
+ * launch's own splits are at most that many, in whole 32-row chunks. Host-only, no device work. No
  * counterpart in the reference.
  */
 int64_t ckv_attention_workspace_bytes(int32_t n_queries, int32_t n_tokens, int32_t n_q_heads,
